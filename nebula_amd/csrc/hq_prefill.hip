@@ -30,7 +30,7 @@ namespace hq {
 namespace {
 
 constexpr int kTilesPerWave = 4;  // 64 columns per wavefront, 256 per workgroup
-// fp16 128-row tiles order each k-block's instructions explicitly (see step()): the LDS
+// fp16 and ternary 128-row tiles order each k-block's instructions explicitly (see step()): the LDS
 // read of A fragment i + kReadAhead issues before the MFMAs of fragment i, and the next
 // chunk's dequantisation is spread between the MFMAs, kValuPerFrag VALU instructions after
 // each fragment's four (the first chunk's, kValuFirst of them, come first). Measured on
@@ -39,6 +39,20 @@ constexpr int kTilesPerWave = 4;  // 64 columns per wavefront, 256 per workgroup
 constexpr int kReadAhead = 3;
 constexpr int kValuFirst = 32;
 constexpr int kValuPerFrag = 7;
+
+// Ternary weights with bf16 activations: t * s rounds to t times the bf16 rounding of the fp16
+// scale s (t is -1, 0 or 1), so a group has one bf16 pattern P to place under its signs.
+// Read as fp16, P is an ordinary number (the exponents of fp16 values in bf16, 103..142, give
+// fp16 exponent fields 12..17), so v_pk_mul_f16 of the fields' +-2.0 by "half of P" (P - 0x400:
+// one less in the exponent field) gives +-P exactly. Both halves of the result hold P - 0x400
+// (0 for a zero scale). Forming t * s in fp32 and rounding each weight took 28 VALU
+// instructions per fragment against 12, the same bits; the 128-row tiles also run fp16's
+// explicit instruction order (5120 x 34816 in bf16, M = 333: 138.4 -> 122.9 us on MI355X).
+__device__ __forceinline__ uint32_t tern_scale_bf16(uint32_t s_f16) {
+  const uint32_t p = f32_to_out<HQ_DTYPE_BF16>(f16_to_f32((uint16_t)s_f16));
+  const uint32_t h = (p & 0x7FFFu) ? p - 0x400u : 0u;
+  return h | (h << 16);
+}
 
 // Dequantised B fragment with the group scale applied. s2 holds the fp16 scale twice.
 // GEN (int4): `add` is the weight of code 8, e = 8 s + b, as fp16 bits (fp16 activations) or
@@ -63,11 +77,19 @@ __device__ __forceinline__ u4 dq_scaled(const u4& w, int c, uint32_t s_f16, cons
     }
     return u4{h2_bits(bits_h2(q[0]) * s2), h2_bits(bits_h2(q[1]) * s2), h2_bits(bits_h2(q[2]) * s2),
               h2_bits(bits_h2(q[3]) * s2)};
+  } else if constexpr (FMT == HQ_FORMAT_TERNARY2) {
+    // s_f16 holds tern_scale_bf16(s) twice: 2t times it in fp16 arithmetic is t times the bf16
+    // scale, bit for bit (one v_pk_mul_f16 per word, as with fp16 activations).
+    const uint32_t word = w[c >> 1];
+    const u4 q = (c & 1) ? dq_tern2<1>(word) : dq_tern2<0>(word);
+    const h2 s2 = bits_h2(s_f16);
+    return u4{h2_bits(bits_h2(q[0]) * s2), h2_bits(bits_h2(q[1]) * s2), h2_bits(bits_h2(q[2]) * s2),
+              h2_bits(bits_h2(q[3]) * s2)};
   } else {
     // No packed bf16 arithmetic on gfx950: form w * s in fp32, round pairs with v_cvt_pk_bf16_f32.
     const float s = f16_to_f32((uint16_t)s_f16);
     float v[8];
-    if constexpr (FMT == HQ_FORMAT_INT4) {
+    {
       const uint32_t x = w[c];
       const uint32_t lo = x & 0x0F0F0F0Fu, hi = (x >> 4) & 0x0F0F0F0Fu;
       // byte b of lo holds element {0,4,1,5}[b], of hi element {2,6,3,7}[b] (nibble order of hq_layout.hpp)
@@ -80,15 +102,6 @@ __device__ __forceinline__ u4 dq_scaled(const u4& w, int c, uint32_t s_f16, cons
       v[6] = __builtin_fmaf((float)((hi >> 8) & 0xFFu), s, ms);
       v[3] = __builtin_fmaf((float)((hi >> 16) & 0xFFu), s, ms);
       v[7] = __builtin_fmaf((float)((hi >> 24) & 0xFFu), s, ms);
-    } else {
-      const uint32_t word = w[c >> 1];
-      const u4 q = (c & 1) ? dq_tern2<1>(word) : dq_tern2<0>(word);  // bf16 bits of 2t
-      const float hs = 0.5f * s;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __builtin_bit_cast(float, q[i] << 16) * hs;
-        v[2 * i + 1] = __builtin_bit_cast(float, q[i] & 0xFFFF0000u) * hs;
-      }
     }
     u4 r;
 #pragma unroll
@@ -145,7 +158,7 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
   // 128-column tiles keep the compiler's order (the explicit one, scaled to two column tiles,
   // measured 6-13% slower) with a ring of two k-blocks (three: 1-3.5% slower, int4 fp16 within
   // 0.5%).
-  constexpr bool kOrdered = DT == HQ_DTYPE_F16 && RT == 8 && !GEN && TW == 4;
+  constexpr bool kOrdered = (DT == HQ_DTYPE_F16 || FMT == HQ_FORMAT_TERNARY2) && RT == 8 && !GEN && TW == 4;
   constexpr int kRing = kOrdered || TW == 2 ? 2 : 3;
   // Partial tiles are stored and loaded with the sc1 cache policy: agent-coherent, so a
   // store that has completed is visible to loads from any XCD.
@@ -375,6 +388,10 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
 #pragma unroll
         for (int t = 0; t < kTilesPerWave; ++t)
           sc[t] = FMT == HQ_FORMAT_TERNARY2 && (sr[slot][t] & 0x7C00u) == 0x7C00u ? 0u : sr[slot][t];
+        if constexpr (FMT == HQ_FORMAT_TERNARY2 && DT == HQ_DTYPE_BF16) {
+#pragma unroll
+          for (int t = 0; t < kTilesPerWave; ++t) sc[t] = tern_scale_bf16(sc[t]);
+        }
         // GEN: chunk c's scale and addend of tile t come from lane 16 c + c16 of the loads.
         uint32_t gsc[GEN ? 4 : 1][kTilesPerWave], gadd[GEN ? 4 : 1][kTilesPerWave];
         if constexpr (GEN) {
@@ -382,7 +399,9 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
           for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int t = 0; t < kTilesPerWave; ++t) {
-              const uint32_t sv = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)sc[t]) & 0xFFFFu;
+              constexpr bool kPairScale = FMT == HQ_FORMAT_TERNARY2 && DT == HQ_DTYPE_BF16;  // tern_scale_bf16: both halves
+              const uint32_t sv = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)sc[t]) &
+                                  (kPairScale ? 0xFFFFFFFFu : 0xFFFFu);
               const uint32_t bv = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)br[slot][t]);
               gsc[c][t] = sv;
               if constexpr (FMT == HQ_FORMAT_INT4) {
