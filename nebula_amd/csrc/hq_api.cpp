@@ -524,9 +524,15 @@ std::string describe(int fmt, int dtype, const hq::GemmDesc& d, const Plan& p) {
                           d.gen ? ",general" : "");
     for (int i = 0; i < p.pc.n && n > 0 && (size_t)n < sizeof b; ++i) {
       const hq::PrefillLaunch& l = p.pc.l[i];
-      n += std::snprintf(b + n, sizeof b - n, "%s launch %d: %u-row%s tiles=%u whole=%u stream-K workgroups=%u%s",
-                         i ? ";" : "", i, 16u * l.RT * l.WM, l.TW == 2 ? " 128-column" : "", l.tiles, l.dp, l.psk,
-                         l.KS == 2 ? " k-split in workgroup" : "");
+      // Tile names: the height alone (256 columns), "128-row 128-column", "64x128".
+      char tile[32];
+      if (l.TW == 2 && l.RT == 4) std::snprintf(tile, sizeof tile, "64x128");
+      else std::snprintf(tile, sizeof tile, "%u-row%s", 16u * l.RT * l.WM, l.TW == 2 ? " 128-column" : "");
+      n += std::snprintf(b + n, sizeof b - n, "%s launch %d: %s tiles=%u whole=%u stream-K workgroups=%u%s", i ? ";" : "",
+                         i, tile, l.tiles, l.dp, l.psk,
+                         l.KS == 4   ? " four-way k-split in workgroup"
+                         : l.KS == 2 ? " k-split in workgroup"
+                                     : "");
     }
     if (n > 0 && (size_t)n < sizeof b) std::snprintf(b + n, sizeof b - n, " ws=%zu", p.need);
   }

@@ -146,7 +146,7 @@ hipError_t launch_decode_ls(int fmt, int dtype, GemmDesc d, const LsConfig& c, v
 struct PrefillLaunch {
   int RT;
   int WM;
-  int KS;  // 2: each tile's k-blocks split between two halves of one workgroup (whole tiles)
+  int KS;  // 2, 4: each tile's k-blocks split between that many groups of four wavefronts (whole tiles)
   int TW;  // column tiles per wavefront: 4 (256-column tiles) or 2 (128-column whole tiles)
   GemmDesc d;
   uint32_t tiles;

@@ -1,10 +1,10 @@
-// hq_prefill.hip — compute-bound qGEMM for M > 16 (prefill, split-fuse batches), gfx950.
+// hq_prefill.hip — compute-bound qGEMM for prefill chunks and larger batches (M > 80), gfx950.
 //
 // The reference has no prefill GEMM (hydrogen's decoder feeds prompt tokens one at a
 // time, native_decoder.cu:1297); this is the MFMA path the target operator asks for.
 //
-// Workgroup tile: (16 * RT * WM) rows x 256 columns, K stepped one 128-deep k-block at a
-// time. 4 * WM wavefronts: WM along M, 4 along N; each owns 16 * RT rows and 64 columns
+// Workgroup tile: (16 * RT * WM) rows x 64 TW columns (256, or 128 with TW = 2), K stepped one
+// 128-deep k-block at a time, in KS groups of wavefronts that split the k-blocks. 4 * WM wavefronts: WM along M, 4 along N; each owns 16 * RT rows and 64 columns
 // (4 column tiles, 16 * RT * 4 fp32 accumulators). A weight fragment is dequantised with
 // its group scale folded in by the WM wavefronts sharing its columns and reused by RT
 // MFMAs each; WM = 2 gives two waves per SIMD so one's dequantisation hides under the
@@ -55,12 +55,13 @@ __device__ __forceinline__ uint32_t tern_scale_bf16(uint32_t s_f16) {
 }
 
 // Dequantised B fragment with the group scale applied. s2 holds the fp16 scale twice.
-// GEN (int4): `add` is the weight of code 8, e = 8 s + b, as fp16 bits (fp16 activations) or
-// the bias b as fp32 bits (bf16 activations), so that the fragment is q * s + b.
+// GEN (int4): the upper half of s_f16 holds the weight of code 8, e = 8 s + b (fp16 activations),
+// or `add` the bias b as fp32 bits (bf16 activations), so that the fragment is q * s + b.
 template <int FMT, int DT, bool GEN = false>
 __device__ __forceinline__ u4 dq_scaled(const u4& w, int c, uint32_t s_f16, const DqConst& k, uint32_t add = 0) {
   if constexpr (DT == HQ_DTYPE_F16) {
-    const h2 s2 = bits_h2(s_f16 | (s_f16 << 16));
+    const h2 sa = bits_h2(s_f16);  // GEN: scale, addend
+    const h2 s2 = {sa[0], sa[0]};
     u4 q;
     if constexpr (FMT == HQ_FORMAT_INT4) {
       q = dq_int4_f16(w[c], k);  // exact q - 8
@@ -69,7 +70,7 @@ __device__ __forceinline__ u4 dq_scaled(const u4& w, int c, uint32_t s_f16, cons
       q = (c & 1) ? dq_tern2<1>(word) : dq_tern2<0>(word);  // exact 2t; the epilogue halves
     }
     if constexpr (GEN && FMT == HQ_FORMAT_INT4) {
-      const h2 e2 = bits_h2(add | (add << 16));
+      const h2 e2 = {sa[1], sa[1]};
       return u4{h2_bits(__builtin_elementwise_fma(bits_h2(q[0]), s2, e2)),
                 h2_bits(__builtin_elementwise_fma(bits_h2(q[1]), s2, e2)),
                 h2_bits(__builtin_elementwise_fma(bits_h2(q[2]), s2, e2)),
@@ -136,17 +137,16 @@ __device__ __forceinline__ void tile_geom(const GemmDesc& d, uint32_t nb, uint32
 // registers never weigh on the whole-tile pipeline.
 // One-row-wave 128-row tiles are held to 256 VGPRs so that two workgroups share a CU (their
 // barriers are independent, so one's dequantisation overlaps the other's MFMAs).
-// GEN: the general kernels (one scale per 32-wide k chunk, optional int4 bias), 64-row tiles.
-// KS = 2 (whole 128-row tiles only): the workgroup's eight wavefronts are two halves of four,
-// each computing the tile over half of its k-blocks through its own LDS stages; the halves'
-// sums meet in LDS at the end (half 0 + half 1). A grid of one tile per CU then still keeps
-// two wavefronts on every SIMD, as two workgroups per CU do.
+// GEN: the general kernels (one scale per 32-wide k chunk, optional int4 bias).
+// KS = 2 or 4 (whole tiles only): the workgroup has KS groups of four wavefronts, each computing
+// the tile over its share of the k-blocks through its own LDS stages; the groups' sums meet in
+// LDS at the end, in group order. A grid of one tile per CU then still keeps two or four
+// wavefronts on every SIMD, as several workgroups per CU do.
 template <int FMT, int DT, int RT, int WM, bool SKP, bool GEN = false, int KS = 1, int TW = 4>
 __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ? 2 : 1)
     hq_prefill_kernel(const GemmDesc d, const PrefillPlan pp) {
-  static_assert(KS == 1 || (KS == 2 && !SKP && !GEN && WM == 1), "the K split is for whole fast tiles");
-  static_assert(TW == 4 || (TW == 2 && KS == 1 && !SKP && !GEN && WM == 1 && RT == 8),
-                "128-column tiles are whole 128-row fast tiles");
+  static_assert(KS == 1 || (!SKP && WM == 1), "the K split is for whole tiles");
+  static_assert(TW == 4 || (TW == 2 && !SKP && WM == 1), "128-column tiles are whole tiles");
   // Column tiles per wavefront: 4 (256-column workgroup tiles) or 2 (128 columns).
   constexpr int kTilesPerWave = TW;
   constexpr uint32_t BM = 16u * RT * WM;
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
   // measured 6-13% slower) with a ring of two k-blocks (three: 1-3.5% slower, int4 fp16 within
   // 0.5%).
   constexpr bool kOrdered = (DT == HQ_DTYPE_F16 || FMT == HQ_FORMAT_TERNARY2) && RT == 8 && !GEN && TW == 4;
-  constexpr int kRing = kOrdered || TW == 2 ? 2 : 3;
+  constexpr int kRing = kOrdered || TW == 2 || (GEN && RT == 8) ? 2 : 3;
   // Partial tiles are stored and loaded with the sc1 cache policy: agent-coherent, so a
   // store that has completed is visible to loads from any XCD.
   constexpr int kCoherent = 16;
@@ -178,18 +178,18 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
 
   const uint32_t bid = blockIdx.x;
 
-  // KS = 2: the two K halves meet separately at every k-block, so that the wavefronts sharing
-  // a SIMD (one per half) drift apart and hide each other's waits (a workgroup barrier kept
+  // KS > 1: the K groups meet separately at every k-block, so that the wavefronts sharing
+  // a SIMD (one per group) drift apart and hide each other's waits (a workgroup barrier kept
   // them in step: the fused QKV tile ran at half the MFMA rate of two independent workgroups
-  // on a CU). A half's barrier is an LDS arrival count (sh_last[kh]): each wavefront adds one
+  // on a CU). A group's barrier is an LDS arrival count (sh_last[kh]): each wavefront adds one
   // once its own copies of the k-block have landed and its reads of the previous stage are
-  // done, and waits until the half's four have arrived. The wait is bounded: every wavefront
-  // of a half executes the same steps, so a correct launch never reaches the bound; one that
+  // done, and waits until the group's four have arrived. The wait is bounded: every wavefront
+  // of a group executes the same steps, so a correct launch never reaches the bound; one that
   // gives up sets the host-visible fault word (reported as HQ_ERR_DEVICE) and carries on.
   uint32_t arrivals = 0;
   const uint32_t harr = (uint32_t)(uintptr_t)(sh_last + kh);
   if constexpr (KS > 1) {
-    if (threadIdx.x < 2u) sh_last[threadIdx.x] = 0u;
+    if (threadIdx.x < (uint32_t)KS) sh_last[threadIdx.x] = 0u;
     __syncthreads();
   }
   auto kblock_barrier = [&]() {
@@ -392,27 +392,34 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
 #pragma unroll
           for (int t = 0; t < kTilesPerWave; ++t) sc[t] = tern_scale_bf16(sc[t]);
         }
-        // GEN: chunk c's scale and addend of tile t come from lane 16 c + c16 of the loads.
+        // GEN: chunk c's scale and addend of tile t come from lane 16 c + c16 of the loads. With
+        // fp16 activations the lane packs both (scale low, addend high) before they travel.
         uint32_t gsc[GEN ? 4 : 1][kTilesPerWave], gadd[GEN ? 4 : 1][kTilesPerWave];
         if constexpr (GEN) {
+          uint32_t own[kTilesPerWave], own_b[kTilesPerWave];
+#pragma unroll
+          for (int t = 0; t < kTilesPerWave; ++t) {
+            own[t] = sc[t];
+            own_b[t] = 0u;
+            if constexpr (FMT == HQ_FORMAT_INT4) {
+              const float s32 = f16_to_f32((uint16_t)sc[t]);
+              if constexpr (DT == HQ_DTYPE_F16) {  // e = 8 s + b (0 without a bias), as fp16
+                if (has_bias)
+                  own[t] = (sc[t] & 0xFFFFu) | ((uint32_t)f32_to_out<HQ_DTYPE_F16>(__builtin_fmaf(
+                                                    8.0f, s32, __builtin_bit_cast(float, br[slot][t]))) << 16);
+              } else {  // the bias b (or -8 s), fp32
+                own_b[t] = has_bias ? br[slot][t] : __builtin_bit_cast(uint32_t, -8.0f * s32);
+              }
+            }
+          }
 #pragma unroll
           for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int t = 0; t < kTilesPerWave; ++t) {
-              constexpr bool kPairScale = FMT == HQ_FORMAT_TERNARY2 && DT == HQ_DTYPE_BF16;  // tern_scale_bf16: both halves
-              const uint32_t sv = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)sc[t]) &
-                                  (kPairScale ? 0xFFFFFFFFu : 0xFFFFu);
-              const uint32_t bv = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)br[slot][t]);
-              gsc[c][t] = sv;
-              if constexpr (FMT == HQ_FORMAT_INT4) {
-                const float s32 = f16_to_f32((uint16_t)sv);
-                if constexpr (DT == HQ_DTYPE_F16)  // e = 8 s + b (0 without a bias), as fp16
-                  gadd[c][t] = has_bias ? f32_to_out<HQ_DTYPE_F16>(__builtin_fmaf(8.0f, s32, __builtin_bit_cast(float, bv))) : 0u;
-                else  // the bias b (or -8 s), fp32
-                  gadd[c][t] = has_bias ? bv : __builtin_bit_cast(uint32_t, -8.0f * s32);
-              } else {
-                gadd[c][t] = 0u;
-              }
+              gsc[c][t] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)own[t]);
+              gadd[c][t] = FMT == HQ_FORMAT_INT4 && DT == HQ_DTYPE_BF16
+                               ? (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)own_b[t])
+                               : 0u;
             }
         }
 #pragma unroll
@@ -485,23 +492,28 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
       __syncthreads();  // the output goes through the activation stages' LDS
       store_tile(s, m0, ct0);
     } else {
-      // Halves of equal length (nkb even, checked by the host), so both meet every barrier.
-      const uint32_t kmid = nkb / 2u;
-      run_piece(s, m0, ct0, kh ? kmid : 0u, kh ? nkb : kmid);
-      __syncthreads();  // both halves are done reading their stages
+      // K group kh takes k-blocks [kh nkb / KS, (kh + 1) nkb / KS); the groups' sums meet in LDS
+      // in group order.
+      run_piece(s, m0, ct0, kh * nkb / KS, (kh + 1u) * nkb / KS);
+      __syncthreads();  // every group is done reading its stages
       f4* const part = reinterpret_cast<f4*>(smem) + wave * (RT * kTilesPerWave * 64u);
+      constexpr uint32_t kGroupPart = 4u * WM * RT * kTilesPerWave * 64u;  // one group's sums
       if (kh) {
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-          for (int t = 0; t < kTilesPerWave; ++t) part[(r * kTilesPerWave + t) * 64u + lane] = acc[r][t];
+          for (int t = 0; t < kTilesPerWave; ++t)
+            part[(kh - 1u) * kGroupPart + (r * kTilesPerWave + t) * 64u + lane] = acc[r][t];
       }
       __syncthreads();
       if (!kh) {
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
+        for (uint32_t k = 0; k + 1u < (uint32_t)KS; ++k)
 #pragma unroll
-          for (int t = 0; t < kTilesPerWave; ++t) acc[r][t] += part[(r * kTilesPerWave + t) * 64u + lane];
+          for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < kTilesPerWave; ++t)
+              acc[r][t] += part[k * kGroupPart + (r * kTilesPerWave + t) * 64u + lane];
       }
       __syncthreads();  // every partial is read before the output reuses the LDS
       if (!kh) store_tile(s, m0, ct0);
@@ -682,48 +694,29 @@ hipError_t launch_rt(const PrefillLaunch& c, void* ws, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Whole 128-row tiles with the K split inside the workgroup (KS = 2): one tile per workgroup.
-template <int FMT, int DT>
-hipError_t launch_ks2(const PrefillLaunch& c, uint32_t* fault, uint32_t spin, hipStream_t stream) {
+// Whole tiles of 16 RT rows x 64 TW columns, one per workgroup, with their k-blocks split
+// between KS groups of four wavefronts.
+template <int FMT, int DT, int RT, int KS, int TW, bool GEN = false>
+hipError_t launch_whole(const PrefillLaunch& c, uint32_t* fault, uint32_t spin, hipStream_t stream) {
+  constexpr uint32_t BM = 16u * RT;
   GemmDesc d = c.d;
   PrefillPlan pp{};
   pp.fault = fault;
   pp.spin = spin;
-  pp.nb = assign_blocks(d);
-  if ((d.M + 127u) / 128u * pp.nb != c.tiles || c.psk != 0 || c.dp != c.tiles || d.nkb % 2u != 0 || d.nkb < 2u)
+  pp.nb = assign_blocks(d, TW);
+  if ((d.M + BM - 1u) / BM * pp.nb != c.tiles || c.psk != 0 || c.dp != c.tiles || d.nkb < (uint32_t)KS)
     return hipErrorInvalidValue;
   pp.dp = c.dp;
   pp.xcd = c.dp % 8u == 0u ? 1u : 0u;
-  pp.bands = (d.M + 127u) / 128u;
+  pp.bands = (d.M + BM - 1u) / BM;
   pp.gb = (uint32_t)std::max(1, env_int("HQ_PREFILL_GB", 4));
   pp.nkb_m = plan_div_magic(d.nkb);
-  const size_t lds = prefill_lds<FMT, DT, 8, 1, 2>();
+  const size_t lds = prefill_lds<FMT, DT, RT, 1, KS>();
   static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_prefill_kernel<FMT, DT, 8, 1, false, false, 2>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_prefill_kernel<FMT, DT, RT, 1, false, GEN, KS, TW>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((hq_prefill_kernel<FMT, DT, 8, 1, false, false, 2>), dim3(c.dp), dim3(512), lds, stream, d, pp);
-  return hipGetLastError();
-}
-
-// Whole 128-row x 128-column tiles (TW = 2): one workgroup per tile, two per CU.
-template <int FMT, int DT>
-hipError_t launch_tw2(const PrefillLaunch& c, hipStream_t stream) {
-  GemmDesc d = c.d;
-  PrefillPlan pp{};
-  pp.nb = assign_blocks(d, 2);
-  if ((d.M + 127u) / 128u * pp.nb != c.tiles || c.psk != 0 || c.dp != c.tiles) return hipErrorInvalidValue;
-  pp.dp = c.dp;
-  pp.xcd = c.dp % 8u == 0u ? 1u : 0u;
-  pp.bands = (d.M + 127u) / 128u;
-  pp.gb = (uint32_t)std::max(1, env_int("HQ_PREFILL_GB", 4));
-  pp.nkb_m = plan_div_magic(d.nkb);
-  const size_t lds = prefill_lds<FMT, DT, 8, 1>();
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_prefill_kernel<FMT, DT, 8, 1, false, false, 1, 2>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((hq_prefill_kernel<FMT, DT, 8, 1, false, false, 1, 2>), dim3(c.dp), dim3(256), lds, stream, d, pp);
+  hipLaunchKernelGGL((hq_prefill_kernel<FMT, DT, RT, 1, false, GEN, KS, TW>), dim3(c.dp), dim3(256 * KS), lds, stream, d, pp);
   return hipGetLastError();
 }
 
@@ -771,9 +764,28 @@ int prefill_slots(int fmt, int RT, int WM) {
 
 template <int FMT, int DT>
 hipError_t launch_fd(const PrefillLaunch& c, void* ws, uint32_t* fault, uint32_t spin, hipStream_t stream) {
+  if (c.WM == 1 && c.psk == 0 && (c.KS > 1 || c.TW == 2 || (c.d.gen && c.RT == 8))) {
+    const int k = c.RT * 100 + c.KS * 10 + c.TW;
+    if (c.d.gen) {
+      switch (k) {
+        case 422: return launch_whole<FMT, DT, 4, 2, 2, true>(c, fault, spin, stream);
+        case 442: return launch_whole<FMT, DT, 4, 4, 2, true>(c, fault, spin, stream);
+        case 814: return launch_whole<FMT, DT, 8, 1, 4, true>(c, fault, spin, stream);
+        case 812: return launch_whole<FMT, DT, 8, 1, 2, true>(c, fault, spin, stream);
+        case 822: return launch_whole<FMT, DT, 8, 2, 2, true>(c, fault, spin, stream);
+      }
+    } else {
+      switch (k) {
+        case 422: return launch_whole<FMT, DT, 4, 2, 2>(c, fault, spin, stream);
+        case 442: return launch_whole<FMT, DT, 4, 4, 2>(c, fault, spin, stream);
+        case 824: return launch_whole<FMT, DT, 8, 2, 4>(c, fault, spin, stream);
+        case 812: return launch_whole<FMT, DT, 8, 1, 2>(c, fault, spin, stream);
+        case 822: return launch_whole<FMT, DT, 8, 2, 2>(c, fault, spin, stream);
+      }
+    }
+    return hipErrorInvalidConfiguration;
+  }
   if (c.d.gen) return c.RT == 4 && c.WM == 1 ? launch_rt<FMT, DT, 4, 1, true>(c, ws, stream) : hipErrorInvalidConfiguration;
-  if (c.KS == 2) return c.RT == 8 && c.WM == 1 ? launch_ks2<FMT, DT>(c, fault, spin, stream) : hipErrorInvalidConfiguration;
-  if (c.TW == 2) return c.RT == 8 && c.WM == 1 ? launch_tw2<FMT, DT>(c, stream) : hipErrorInvalidConfiguration;
   if (c.RT == 4) return launch_rt<FMT, DT, 4, 1>(c, ws, stream);
   if (c.WM == 1) return launch_rt<FMT, DT, 8, 1>(c, ws, stream);
   return launch_rt<FMT, DT, 8, 2>(c, ws, stream);
@@ -952,9 +964,73 @@ bool env_set(const char* name) {
   const char* v = std::getenv(name);
   return v && *v;
 }
+
+PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
+  PrefillLaunch l = make_launch(RT, 1, d, TW);
+  l.KS = KS;
+  return l;
+}
+
+// 128-column whole tiles for grids that are small beside the chip, in place of the plan over
+// 256-column tiles (`cur`), and the general kernels' 128-row tiles for large ones. Such grids
+// left CUs idle or split their tiles along K over workgroups, paying for partial tiles in
+// memory; a 64- or 128-row x 128-column tile per CU whose k-blocks are split between the
+// workgroup's own groups of wavefronts keeps every SIMD busy and adds the groups' sums in LDS.
+// The choice is the same for both activation types (the workspace queries do not know it).
+// Measured on MI355X (K = 4096, previous plan -> this one, int4 fp16 / int4 bf16 / ternary fp16):
+//  * 64 x 128 tiles at most one per CU, four groups: M = 128, N = 14336 (224 tiles) 49.8 -> 23.4 /
+//    52.2 -> 27.3 / 30.5 -> 21.1 us; M = 333, N = 4096 (192) 46.0 -> 20.3 / 46.6 -> 26.4 / 35.4 ->
+//    19.0; M = 81, N = 4096 (64) 24.1 -> 19.4 / 26 -> 25.6 / 24.6 -> 18.5. Their time grows with K
+//    alone, that of a K split over workgroups with the work, so the line rises with K: at 64
+//    k-blocks (K = 8192) 64 tiles 37.4 -> 33.0 but 32 tiles 26.3 -> 32.3; at 216 (K = 27648)
+//    int4 240 tiles 126 -> 114, 120 tiles 92 -> 97, ternary 240 109 -> 104, 120 68 -> 94; at 112
+//    (K = 14336) 128 tiles int4 70 -> 57, ternary 46 -> 52. Below
+//    17 k-blocks two groups do (K = 1024, M = 384, N = 4096: 16.5 -> 8.9 us, four groups 9.7).
+//  * more 64 x 128 tiles, up to two per CU: int4 takes 128 x 128 tiles of two groups while those
+//    fit one per CU (M = 256, N = 14336: 45.8 -> 35.1 us; bf16 M = 333, N = 7168 48.7 -> 38.7,
+//    64 x 128 tiles 45.0), otherwise, and for ternary, 64 x 128 tiles of two groups (M = 192, N =
+//    20480 50.4 -> 39.5 / 56.5 -> 47.8 / 42.5 -> 35.6). At 516 tiles the gain is gone (5 / 0 / 10%).
+//  * the general kernels beyond that: the cheapest of 64 x 128 (two groups), 128 x 128 and 128 x
+//    256 tiles (one group) by rounds, in place of 64-row tiles of 256 columns, whose dequantised
+//    weights serve half the rows (K = 4096, group 32 with a bias: M = 1024, N = 14336 fp16 143 -> 114
+//    us, bf16 183 -> 129, 128 x 256; M = 512, N = 14336 76.0 -> 67.7, 96.5 -> 77.4, 128 x 128; M = 160,
+//    N = 27648 84.7 -> 62.3, 102.8 -> 72.9, 64 x 128).
+bool choose_small_tiles(int fmt, const GemmDesc& d, const PrefillLaunch& cur, PrefillLaunch* out) {
+  if (d.M <= 64u || d.nkb < 4u) return false;
+  for (const char* e : {"HQ_PREFILL_RT", "HQ_PREFILL_WM", "HQ_PREFILL_KS", "HQ_PREFILL_PSK", "HQ_PREFILL_SK", "HQ_PREFILL_TW"})
+    if (env_set(e)) return false;  // a forced plan stays
+  const uint32_t cus = (uint32_t)cu_count();
+  const bool int4 = fmt == HQ_FORMAT_INT4;
+  const uint32_t t64 = make_launch(4, 1, d, 2).tiles, t128 = make_launch(8, 1, d, 2).tiles;
+  if (t64 <= cus) {
+    // Tiles from which the whole tiles win, for 256 CUs.
+    uint32_t from = d.nkb <= 16u ? 32u : int4 && d.nkb > 32u ? 80u : 64u;
+    if (d.nkb > 64u) from += int4 ? (d.nkb - 64u) / 2u : (d.nkb - 64u) * 7u / 5u;
+    if ((uint64_t)t64 * 256u < (uint64_t)from * cus) return false;
+    *out = make_whole(4, d.nkb <= 16u ? 2 : 4, 2, d);
+    return true;
+  }
+  // A long K stays split over workgroups (K = 27648, M = 512, N = 5120: 170 us against 186-199).
+  if (cur.psk != 0 && d.nkb > 64u) return false;
+  if (t64 <= 2u * cus) {
+    *out = int4 && t128 <= cus ? make_whole(8, 2, 2, d) : make_whole(4, 2, 2, d);
+    return true;
+  }
+  if (!d.gen) return false;
+  // Rounds of 512 tiles (two per CU): a last round that leaves every CU at most one tile costs
+  // 0.6 of a round, a fuller one 0.95; a round of the three tiles takes 41 : 71.5 : 119.
+  auto rounds = [&](uint32_t t) {
+    const uint32_t rest = t % (2u * cus);
+    return (double)(t / (2u * cus)) + (rest == 0u ? 0.0 : rest <= cus ? 0.6 : 0.95);
+  };
+  const double c422 = 41.0 * rounds(t64), c812 = 71.5 * rounds(t128), c814 = 119.0 * rounds(make_launch(8, 1, d).tiles);
+  *out = c814 <= c422 && c814 <= c812 ? make_whole(8, 1, 4, d) : c812 <= c422 ? make_whole(8, 1, 2, d) : make_whole(4, 2, 2, d);
+  return true;
+}
 }  // namespace
 
-// The plan over 256-column tiles, then 128-row x 128-column whole tiles (TW = 2, four
+// The plan over 256-column tiles, then the small grids' tiles (choose_small_tiles), then
+// 128-row x 128-column whole tiles (TW = 2, four
 // wavefronts of 32 columns, two workgroups per CU) in place of a one-round whole-tile grid
 // that leaves the CUs one workgroup each or uneven: at the same tile count as 64-row tiles
 // each dequantised weight serves twice the rows, and against a 128-row tile split in two K
@@ -975,7 +1051,21 @@ bool env_set(const char* name) {
 // Stream-K plans (short grids, long K) stay: 128-column tiles there were 1-40% slower.
 PrefillConfig choose_prefill(int fmt, const GemmDesc& d, size_t ws_cap, int dtype) {
   PrefillConfig c = choose_prefill_256(fmt, d, ws_cap);
-  if (d.gen || c.n != 1) return c;
+  if (const int f = env_int("HQ_PREFILL_TILE", 0)) {  // tuning / test override: RT * 100 + KS * 10 + TW
+    const PrefillLaunch l = make_whole(f / 100, f / 10 % 10, f % 10, d);
+    if (d.nkb >= (uint32_t)l.KS) {
+      c.n = 1;
+      c.l[0] = l;
+    }
+    return c;
+  }
+  if (c.n != 1) return c;
+  PrefillLaunch small;
+  if (choose_small_tiles(fmt, d, c.l[0], &small)) {
+    c.l[0] = small;
+    return c;
+  }
+  if (d.gen) return c;
   PrefillLaunch& l = c.l[0];
   const int etw = env_int("HQ_PREFILL_TW", 0);  // tuning / test override: 2 forces, 1 forbids
   if (etw == 2) {
