@@ -147,7 +147,8 @@ hq_status get_internal_ws(hipStream_t stream, size_t need, void** out) {
 // lockstep kernel takes them. With ternary weights the lockstep kernel's
 // four-k-group configuration is faster from one row on (5120 x 27648 at M = 1: 12.8 us
 // against 14.7 us), so it is taken whenever the lockstep planner picks it. The general
-// kernels (bias, groups that are not multiples of 128) exist in the lockstep family only.
+// kernels (bias, groups that are not multiples of 128) exist in the lockstep and (int4) the
+// X-resident family only.
 // HQ_DECODE_KERNEL=0 / 1 forces one of them for M <= 16 (tuning and tests).
 bool use_lockstep(int fmt, const hq::GemmDesc& d) {
   if (d.M > 16 || d.gen) return true;  // only the lockstep kernel takes several row tiles
@@ -158,10 +159,10 @@ bool use_lockstep(int fmt, const hq::GemmDesc& d) {
 }
 
 // The X-resident kernel (hq_decode.hip) takes every call with at most 16 rows whose
-// activation rows fit in LDS, outside the general kernels. HQ_DECODE_KERNEL=2 forces it
+// activation rows fit in LDS, general int4 calls among them. HQ_DECODE_KERNEL=2 forces it
 // where it fits, 0 or 1 keeps it off (tuning and tests).
 bool use_resident(int fmt, const hq::GemmDesc& d, size_t cap, hq::XrConfig* c) {
-  if (d.M > 16 || d.gen) return false;
+  if (d.M > 16) return false;
   const char* v = std::getenv("HQ_DECODE_KERNEL");
   if (v && *v && std::atoi(v) != 2) return false;
   *c = hq::choose_decode_xr(fmt, d, cap);
@@ -506,8 +507,8 @@ std::string describe(int fmt, int dtype, const hq::GemmDesc& d, const Plan& p) {
                   slabs, p.xc.S, p.xc.WK, p.xc.lds, p.need);
   } else if (p.kind == Kind::kResident) {
     std::snprintf(b, sizeof b,
-                  "hq_decode_xr_kernel<%s,%s,T=%d,U=%d> workgroups=%u slabs x %d pieces x %d wavefronts lds=%u ws=%zu",
-                  fmt_name(fmt), dt_name(dtype), p.xc.T, p.xc.U, xr_slabs(d, p.xc.T, p.xc.G), p.xc.S, p.xc.WK, p.xc.lds,
+                  "hq_decode_xr_kernel<%s,%s,T=%d,U=%d%s> workgroups=%u slabs x %d pieces x %d wavefronts lds=%u ws=%zu",
+                  fmt_name(fmt), dt_name(dtype), p.xc.T, p.xc.U, d.gen ? ",general" : "", xr_slabs(d, p.xc.T, p.xc.G), p.xc.S, p.xc.WK, p.xc.lds,
                   p.need);
   } else if (p.kind == Kind::kDecode) {
     std::snprintf(b, sizeof b, "hq_decode_kernel<%s,%s,T=%d,U=%d> workgroups=%d x %d wavefronts%s%s ws=%zu",

@@ -449,15 +449,30 @@ struct XrPlan {
 constexpr int xr_max_wk(int T) { return T >= 8 ? 8 : 16; }
 
 // GRP: slab groups (pl.sg of them per workgroup); without it one slab per workgroup.
-template <int FMT, int DT, int T, int U, bool FUSED, bool GRP = false>
-__global__ void __launch_bounds__(64 * xr_max_wk(T)) hq_decode_xr_kernel(const GemmDesc d, const XrPlan pl) {
+//
+// GEN: the general int4 kernels (one scale per 32-wide k chunk, for groups that are multiples of
+// 32, and an optional fp32 bias per group: w = q * s + b). Load t of a step's scales (and of its
+// biases) gives lane l column 16 (ct0 + t) + l % 16 in chunk l / 16. The chunks' sums are scaled
+// one by one, each lane taking its column's scale of chunk c from lane 16 c + l % 16. With
+// e = 8 s + b (the weight of code 8, in fp32) the bias adds sum_c e_c sum(x over chunk c), a
+// product of the 16 x 4 chunk sums and the 4 x 16 e: one v_mfma_f32_16x16x4_f32 per tile and
+// k-block, whose B operand is the loads' own lane order. The chunk sums in its A order (lane: row
+// l % 16, chunk l / 16) come from four MFMAs against fragments whose rows 4 c .. 4 c + 3 are ones
+// for chunk c. The HBM stream bounds it as it does the fast kernels (Q4_K moves 1,408 bytes per
+// tile and k-block against 1,056); MI355X, 4096 x 14336, group 32, bias, bf16 (lockstep
+// general kernel -> this one): M = 1 / 4 / 16 22.5 / 22.6 / 22.8 -> 12.9 / 13.1 / 14.0 us (three
+// steps in flight 14.5-15.6), 5120 x 5120 M = 4 11.5 -> 9.7, 27648 x 5120 M = 4 29.6 -> 25.9.
+template <int FMT, int DT, int T, int U, bool FUSED, bool GRP = false, bool GEN = false>
+__global__ void __launch_bounds__(GEN ? 512 : 64 * xr_max_wk(T)) hq_decode_xr_kernel(const GemmDesc d, const XrPlan pl) {
   using W = typename WTraits<FMT>::V;
   constexpr uint32_t WPL = WTraits<FMT>::wpl;
   constexpr uint32_t kLaneBytes = WPL * 4u;
   constexpr uint32_t kBlockBytes = 64u * kLaneBytes;  // one tile x one k-block
   constexpr uint32_t kCols = 16u * T;
   constexpr bool kInt4 = FMT == HQ_FORMAT_INT4;
-  constexpr int kSL = (T + 3) / 4;  // scale loads per step (one per four tiles)
+  static_assert(!GEN || kInt4, "the general X-resident kernels are int4");
+  constexpr int kSL = GEN ? T : (T + 3) / 4;  // scale loads per step (one per four tiles; GEN: one per tile)
+  constexpr int kBL = GEN ? T : 0;            // bias loads per step
   extern __shared__ __attribute__((aligned(16))) char xs[];
 
   const uint32_t lane = threadIdx.x & 63u;
@@ -524,17 +539,23 @@ __global__ void __launch_bounds__(64 * xr_max_wk(T)) hq_decode_xr_kernel(const G
   const uint32_t nj = gl && wi < nkbp ? (nkbp - wi + WK - 1u) / WK : 0u;
   const __amdgpu_buffer_rsrc_t wrs =
       make_rsrc(sg.Wp + (size_t)ct0 * nkb * 64u * WPL, __builtin_amdgcn_readfirstlane(nv * nkb * kBlockBytes));
-  const __amdgpu_buffer_rsrc_t srs = make_rsrc(sg.S, __builtin_amdgcn_readfirstlane(((nkb / gkb - 1u) * sg.lds + N) * 2u));
+  const uint32_t srows = GEN ? 4u * nkb / d.g32 : nkb / gkb;
+  const __amdgpu_buffer_rsrc_t srs = make_rsrc(sg.S, __builtin_amdgcn_readfirstlane(((srows - 1u) * sg.lds + N) * 2u));
+  const bool has_bias = GEN && sg.B != nullptr;
+  const __amdgpu_buffer_rsrc_t brs =
+      make_rsrc(sg.B, has_bias ? __builtin_amdgcn_readfirstlane(((srows - 1u) * sg.lds + N) * 4u) : 0u);
   const uint32_t lsrow = sg.lds * 2u;
   uint32_t wvo[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) wvo[t] = lane * kLaneBytes + (uint32_t)t * nkb * kBlockBytes;
   uint32_t svo[kSL];
 #pragma unroll
-  for (int jj = 0; jj < kSL; ++jj) svo[jj] = min(ct0 * 16u + 64u * jj + lane % kCols, N - 1u) * 2u;
+  for (int jj = 0; jj < kSL; ++jj)
+    svo[jj] = GEN ? min((ct0 + jj) * 16u + c16, N - 1u) * 2u : min(ct0 * 16u + 64u * jj + lane % kCols, N - 1u) * 2u;
 
   W wr[U][T];
   uint32_t sr[U][kSL];
+  uint32_t br[U][GEN ? T : 1];
   auto load = [&](int slot, uint32_t j) {
     const bool live = j < nj;
     const uint32_t kb = kb0 + wi + j * WK;
@@ -545,16 +566,27 @@ __global__ void __launch_bounds__(64 * xr_max_wk(T)) hq_decode_xr_kernel(const G
       if constexpr (WPL == 4) wr[slot][t] = __builtin_amdgcn_raw_buffer_load_b128(wrs, live ? wvo[t] : kOutOfRange, kbo, kStreamAux);
       else wr[slot][t] = __builtin_amdgcn_raw_buffer_load_b64(wrs, live ? wvo[t] : kOutOfRange, kbo, kStreamAux);
     }
+    if constexpr (GEN) {
+      // Chunk g4 of k-block kb: scale row (4 kb + g4) / g32, per lane.
+      const uint32_t row = live ? plan_div(4u * kb + g4, d.g32, d.g32_m) : 0u;
 #pragma unroll
-    for (int jj = 0; jj < kSL; ++jj) sr[slot][jj] = __builtin_amdgcn_raw_buffer_load_b16(srs, live ? svo[jj] : kOutOfRange, so, 0);
+      for (int t = 0; t < T; ++t) {
+        const uint32_t o = live ? row * lsrow + svo[t] : kOutOfRange;
+        sr[slot][t] = __builtin_amdgcn_raw_buffer_load_b16(srs, o, 0, 0);
+        br[slot][t] = __builtin_amdgcn_raw_buffer_load_b32(brs, live ? 2u * o : kOutOfRange, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int jj = 0; jj < kSL; ++jj) sr[slot][jj] = __builtin_amdgcn_raw_buffer_load_b16(srs, live ? svo[jj] : kOutOfRange, so, 0);
+    }
   };
 #pragma unroll
   for (int u = 0; u < U; ++u) load(u, (uint32_t)u);
   __builtin_amdgcn_sched_barrier(0);
 
-  // Wait for this wavefront's activation copies only: the ring's U * (T + kSL) loads were
+  // Wait for this wavefront's activation copies only: the ring's U * (T + kSL + kBL) loads were
   // issued after them and stay in flight. Then publish the rows to the workgroup.
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(U * (T + kSL)));
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(U * (T + kSL + kBL)));
   __syncthreads();
 
   // A fragment addresses: a[c] = xa[c] + (kb - kb0) * 256.
@@ -568,6 +600,45 @@ __global__ void __launch_bounds__(64 * xr_max_wk(T)) hq_decode_xr_kernel(const G
   f4 acc[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+
+  // GEN: fragment c of the chunk sums, rows 4 c .. 4 c + 3 ones.
+  constexpr uint32_t one2 = DT == HQ_DTYPE_F16 ? 0x3C003C00u : 0x3F803F80u;
+  auto compute_gen = [&](int u, uint32_t j) {
+    const uint32_t kbl = wi + j * WK;
+    u4 a[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) a[c] = *reinterpret_cast<const u4*>(xs + xa[c] + kbl * 256u);
+    uint32_t sb[GEN ? T : 1][4];
+#pragma unroll
+    for (int t = 0; t < (GEN ? T : 1); ++t)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        sb[t][c] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((16u * c + c16) * 4u), (int)sr[u][t]);
+    if (has_bias) {  // uniform
+      f4 sx = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint32_t o = (c16 >> 2) == (uint32_t)c ? one2 : 0u;
+        sx = mfma16x16x32<DT>(u4{o, o, o, o}, a[c], sx);
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const float e = __builtin_fmaf(8.0f, f16_to_f32((uint16_t)sr[u][GEN ? t : 0]), __builtin_bit_cast(float, br[u][GEN ? t : 0]));
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[0], e, acc[t], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const f4 seed = mfma16x16x32<DT>(a[c], corr_b, f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const f4 gs = mfma16x16x32<DT>(a[c], dq_int4_biased<DT>(wr[u][t][c], dqb), seed);
+        const float sc = f16_to_f32((uint16_t)sb[GEN ? t : 0][c]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[t][v] = __builtin_fmaf(gs[v], sc, acc[t][v]);
+      }
+    }
+  };
 
   auto compute = [&](int u, uint32_t j) {
     const uint32_t kbl = wi + j * WK;  // k-block within the piece
@@ -625,7 +696,10 @@ __global__ void __launch_bounds__(64 * xr_max_wk(T)) hq_decode_xr_kernel(const G
   for (uint32_t j = 0; j < nj; j += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (j + u < nj) compute(u, j + u);  // uniform; no loads inside, so waitcnt stays exact across it
+      if (j + u < nj) {  // uniform; no loads inside, so waitcnt stays exact across it
+        if constexpr (GEN) compute_gen(u, j + u);
+        else compute(u, j + u);
+      }
       load(u, j + u + U);
     }
   }
@@ -948,9 +1022,9 @@ uint32_t xr_lds_bytes(const GemmDesc& d, int T, int WK, int S, int SG = 1) {
   return std::max(x, red);
 }
 
-template <int FMT, int DT, int T, int U, bool GRP = false>
+template <int FMT, int DT, int T, int U, bool GRP = false, bool GEN = false>
 hipError_t xr_launch_t(GemmDesc d, const XrConfig& c, void* ws, hipStream_t stream) {
-  if (c.WK < 1 || c.SG < 1 || c.WK * c.SG > xr_max_wk(T) || d.M > 16u || c.S < 1 || (uint32_t)c.S > d.nkb ||
+  if ((GEN && c.WK > 8) || c.WK < 1 || c.SG < 1 || c.WK * c.SG > xr_max_wk(T) || d.M > 16u || c.S < 1 || (uint32_t)c.S > d.nkb ||
       (c.SG > 1 && (c.S > 1 || !GRP)))
     return hipErrorInvalidValue;
   const uint32_t G = assign_slabs(d, T, c.G);
@@ -977,24 +1051,34 @@ hipError_t xr_launch_t(GemmDesc d, const XrConfig& c, void* ws, hipStream_t stre
     fits = fits && (uint64_t)(d.seg[i].slab_w + 1u) * d.nkb * 64u * WTraits<FMT>::wpl * 4u < (1ull << 31);
   if (!fits) return hipErrorInvalidValue;
   static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_decode_xr_kernel<FMT, DT, T, U, false, GRP>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_decode_xr_kernel<FMT, DT, T, U, false, GRP, GEN>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kXrLdsMax) != hipSuccess
           ? hipErrorInvalidConfiguration
-          : hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_decode_xr_kernel<FMT, DT, T, U, true, GRP>),
+          : hipFuncSetAttribute(reinterpret_cast<const void*>(&hq_decode_xr_kernel<FMT, DT, T, U, true, GRP, GEN>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kXrLdsMax);
   if (attr != hipSuccess) return attr;
   const dim3 grid(GW, pl.S);
   if (d.nseg > 1)
-    hipLaunchKernelGGL((hq_decode_xr_kernel<FMT, DT, T, U, true, GRP>), grid, dim3(64 * c.WK * c.SG), c.lds, stream, d,
+    hipLaunchKernelGGL((hq_decode_xr_kernel<FMT, DT, T, U, true, GRP, GEN>), grid, dim3(64 * c.WK * c.SG), c.lds, stream, d,
                        pl);
   else
-    hipLaunchKernelGGL((hq_decode_xr_kernel<FMT, DT, T, U, false, GRP>), grid, dim3(64 * c.WK * c.SG), c.lds, stream,
+    hipLaunchKernelGGL((hq_decode_xr_kernel<FMT, DT, T, U, false, GRP, GEN>), grid, dim3(64 * c.WK * c.SG), c.lds, stream,
                        d, pl);
   return hipGetLastError();
 }
 
 template <int FMT, int DT>
 hipError_t xr_launch_fd(const GemmDesc& d, const XrConfig& c, void* ws, hipStream_t stream) {
+  if (d.gen) {
+    if constexpr (FMT == HQ_FORMAT_INT4) {
+      switch (c.T * 10 + c.U) {
+        case 42: return xr_launch_t<FMT, DT, 4, 2, false, true>(d, c, ws, stream);
+        case 23: return xr_launch_t<FMT, DT, 2, 3, false, true>(d, c, ws, stream);
+        case 14: return xr_launch_t<FMT, DT, 1, 4, false, true>(d, c, ws, stream);
+      }
+    }
+    return hipErrorInvalidConfiguration;
+  }
   switch (c.T * 10 + c.U) {
     case 82: return xr_launch_t<FMT, DT, 8, 2>(d, c, ws, stream);
     case 42:
@@ -1069,10 +1153,18 @@ static int xr_waves_per_simd(int fmt, int T, int U) {
 // HQ_XR_T / _WK / _U / _S / _G (slab count) / _SG (slab groups per workgroup) override (tuning and tests).
 XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   XrConfig c{2, 3, 8, 1, 0, false};
-  if (d.M > 16u || d.gen) return c;
+  if (d.M > 16u || (d.gen && fmt != HQ_FORMAT_INT4)) return c;
   const uint32_t cus = (uint32_t)cu_count();
   uint32_t tiles = 0;
   for (uint32_t i = 0; i < d.nseg; ++i) tiles += d.seg[i].ntiles;
+  // The general kernels: two wavefronts per SIMD (their registers), no slab groups; not for the few
+  // tiles whose slabs the lockstep kernel cuts along K (N = 256 and below: equal; N = 512, K = 4096:
+  // 7.3 -> 6.1 us here).
+  // Above eight rows a call of at most one tile per CU keeps the lockstep kernel's K pieces and with
+  // them the workspace such calls have always asked for, which grows with the row tiles (one-tile
+  // slabs here: 4096 x 4096 M = 16 9.7 -> 8.4 us, 4096 x 2048 8.9 -> 7.4).
+  if (d.gen && (8u * tiles < cus || (d.M > 8u && tiles <= cus))) return c;
+  auto waves_per_simd = [&](int T, int U) { return d.gen ? 2 : xr_waves_per_simd(fmt, T, U); };
   const int eT = env_int("HQ_XR_T", 0), eWK = env_int("HQ_XR_WK", 0), eU = env_int("HQ_XR_U", 0);
   const int eS = env_int("HQ_XR_S", 0), eG = env_int("HQ_XR_G", 0), eSG = env_int("HQ_XR_SG", 0);
   const bool forced = eT || eWK || eU || eS || eG || eSG;
@@ -1113,6 +1205,7 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
     for (int s = 2; s <= 8; ++s) {
       if ((uint32_t)s > d.nkb || xr_x_bytes(d, s) > kXrLdsMax) continue;
       for (int t : {2, 4, 8}) {
+        if (t == 8 && d.gen) continue;
         const int wk = t == 8 ? 4 : 8, u = t == 2 ? 3 : 2;
         const uint32_t lds = xr_lds_bytes(d, t, wk, s);
         const uint32_t wgs = total_slabs(d, t) * (uint32_t)s;
@@ -1128,6 +1221,7 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   for (int s = 1; s <= 8 && !found; ++s) {
     if ((uint32_t)s > d.nkb || xr_x_bytes(d, s) > kXrLdsMax || (s > 1 && d.M > 4u)) continue;
     for (int t : {1, 2, 4, 8}) {
+      if (t == 8 && d.gen) continue;  // 8-tile slabs of the general kernels do not fit in registers
       // One-tile slabs only when they give every CU at most one (4096 x 4096, M = 16: 256
       // workgroups, 5.96 against 6.55-6.69 us with 2-tile slabs; with more tiles than CUs,
       // 2-tile slabs measured faster: 5120 x 5120, M = 4: 6.08 against 7.14); fewer tiles than
@@ -1138,12 +1232,12 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
       // 12288 / 14336 and 5120 x 13824 5-13% faster (4096 x 11008 M = 1 8.36 -> 7.26 us),
       // ternary 2-12%.
       if (t == 2 && !forced && total_slabs(d, 2) > cus && total_slabs(d, 4) <= cus &&
-          xr_lds_bytes(d, 4, 8, s) <= kXrLdsMax && xr_waves_per_simd(fmt, 4, 2) >= 2)
+          xr_lds_bytes(d, 4, 8, s) <= kXrLdsMax && waves_per_simd(4, 2) >= 2)
         continue;
       const int wk = t == 8 ? 4 : 8, u = t == 1 ? 4 : t == 2 ? 3 : 2;
       const uint32_t lds = xr_lds_bytes(d, t, wk, s);
       if (lds > kXrLdsMax) continue;
-      const uint32_t by_regs = (uint32_t)(xr_waves_per_simd(fmt, t, u) / ((wk + 3) / 4));
+      const uint32_t by_regs = (uint32_t)(waves_per_simd(t, u) / ((wk + 3) / 4));
       const uint32_t per_cu = std::min(by_regs, kXrLdsMax / lds);
       const uint32_t wgs = total_slabs(d, t) * (uint32_t)s;
       // 4-tile slabs up to one and a half rounds beat 8-tile slabs of four wavefronts in one
@@ -1160,7 +1254,7 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
       // 2-8% faster; at four rows, or with 4-tile slabs in one round, no gain.
       if (t == 4 && wgs > cus * per_cu && d.M <= 2u) {
         const uint32_t lds2 = xr_lds_bytes(d, 2, 4, s);
-        const uint32_t per2 = std::min((uint32_t)xr_waves_per_simd(fmt, 2, 3), kXrLdsMax / lds2);
+        const uint32_t per2 = std::min((uint32_t)waves_per_simd(2, 3), kXrLdsMax / lds2);
         if (lds2 <= kXrLdsMax && total_slabs(d, 2) * (uint32_t)s <= cus * per2) {
           c = XrConfig{2, 3, 4, s, lds2, false};
           found = true;
@@ -1174,6 +1268,16 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
       break;
     }
   }
+  // General kernels, more 4-tile slabs than one round takes: two workgroups of four wavefronts per
+  // CU, in as many rounds as it needs, where the rows fit twice (5120 x 27648, M = 4: 30.4 -> 25.4
+  // us; one workgroup per CU loses to the lockstep kernel, M = 16: 29.7-30.3 against 31.3).
+  if (!forced && !found && d.gen && tiles > cus && xr_x_bytes(d, 1) <= kXrLdsMax) {
+    const uint32_t lds = xr_lds_bytes(d, 4, 4, 1);
+    if (2u * lds <= kXrLdsMax && total_slabs(d, 4) <= 65535u) {
+      c = XrConfig{4, 2, 4, 1, lds, false};
+      found = one_round = true;
+    }
+  }
   // Whole 4-tile slabs at up to eight rows, more of them than CUs: four wavefronts (one per
   // SIMD, each streaming twice the k-blocks) instead of eight, when that grid still fits on the
   // CUs in one round. Measured on MI355X (alternated runs): 5120 x 27648 int4 M = 1..8
@@ -1182,7 +1286,7 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   // -> 18.7), and so it does with one slab per CU (4096 x 14336, 224 slabs: 8.26 -> 8.49 us).
   if (!forced && found && c.T == 4 && c.WK == 8 && c.S == 1 && d.M <= 8u && total_slabs(d, 4) > cus) {
     const uint32_t lds4 = xr_lds_bytes(d, 4, 4, 1);
-    const uint32_t per4 = std::min((uint32_t)xr_waves_per_simd(fmt, 4, 2), kXrLdsMax / lds4);
+    const uint32_t per4 = std::min((uint32_t)waves_per_simd(4, 2), kXrLdsMax / lds4);
     if (lds4 <= kXrLdsMax && per4 >= 1u && total_slabs(d, 4) <= cus * per4) {
       c.WK = 4;
       c.lds = lds4;
@@ -1205,12 +1309,12 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   // instead (5120 x 27648 M = 1: 11.7 -> 12.3 us in pairs; 272-352 slabs within 3%), and in
   // triples below four rows (M = 1: 11.8 -> 12.6 us); so do one or two rows where 2-tile slabs
   // of four wavefronts fit in one round (above; int4 triples no faster there).
-  if (!forced && xr_x_bytes(d, 1) <= kXrLdsMax && !(found && (c.T < 4 || c.S > 1))) {
+  if (!forced && !d.gen && xr_x_bytes(d, 1) <= kXrLdsMax && !(found && (c.T < 4 || c.S > 1))) {
     const uint32_t sl4 = total_slabs(d, 4);
     const uint32_t sg = (sl4 + cus - 1u) / cus;
     const bool rows_ok = fmt == HQ_FORMAT_INT4 || sg >= 4u || (sg == 3u ? d.M >= 4u : d.M > 8u);
     const uint32_t ldsg = xr_lds_bytes(d, 4, 4, 1, (int)sg);
-    if (sl4 > cus && sg <= 4u && rows_ok && ldsg <= kXrLdsMax && (uint32_t)xr_waves_per_simd(fmt, 4, 2) >= sg) {
+    if (sl4 > cus && sg <= 4u && rows_ok && ldsg <= kXrLdsMax && (uint32_t)waves_per_simd(4, 2) >= sg) {
       c = XrConfig{4, 2, 4, 1, ldsg, false};
       c.SG = (int)sg;
       found = one_round = true;
@@ -1218,7 +1322,7 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   }
   // Wide weights at more than eight rows: the lockstep kernel unless one round of slabs of at
   // most four tiles (eight wavefronts) fits.
-  const bool wide_rows = tiles > 2u * cus && d.M > 8u && (c.T > 4 || !one_round) && c.SG == 1;
+  const bool wide_rows = !d.gen && tiles > 2u * cus && d.M > 8u && (c.T > 4 || !one_round) && c.SG == 1;
   if (!forced && (!found || wide_rows)) return c;
   if (eT == 1 || eT == 2 || eT == 4 || eT == 8) c.T = eT;
   if (eWK >= 1) c.WK = eWK;
@@ -1233,7 +1337,12 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   if (c.T == 1) c.U = c.U >= 6 ? 6 : 4;
   c.WK = std::max(1, std::min(c.WK, xr_max_wk(c.T)));
   c.SG = std::max(1, std::min(c.SG, xr_max_wk(c.T) / c.WK));
-  if (c.S > 1 || c.T != 4) c.SG = 1;  // slab groups: whole 4-tile slabs only
+  if (d.gen) {
+    c.WK = std::min(c.WK, 8);
+    if (c.T == 8) c.T = 4;
+    c.U = c.T == 4 ? 2 : c.T == 2 ? 3 : 4;
+  }
+  if (c.S > 1 || c.T != 4 || d.gen) c.SG = 1;  // slab groups: whole 4-tile slabs only
   c.S = std::max(1, std::min<int>(c.S, (int)d.nkb));
   if (c.G && total_slabs(d, c.T, c.G) > 65535u) return c;
   if (c.S > 1 && (total_slabs(d, c.T, c.G) > kMaxCounters || decode_xr_workspace_bytes(d, c) > ws_cap)) return c;

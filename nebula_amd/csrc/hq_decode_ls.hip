@@ -37,8 +37,8 @@
 // split slab are summed in piece order by the last workgroup to finish (arrival counter),
 // so results are deterministic.
 //
-// General kernels (GEN): one scale per 32-wide k chunk (groups that are multiples of 32, not
-// of 128) and an optional fp32 per-group bias, the reference's w = q * s + b
+// General kernels (GEN; at M <= 16 the X-resident kernel takes most int4 calls): one scale per
+// 32-wide k chunk (groups that are multiples of 32, not of 128) and an optional fp32 per-group bias, the reference's w = q * s + b
 // (marlin_gemm.cu:195-196). With e = 8 s + b (the weight of code 8) the chunk's contribution
 // is s * sum x (q - 8) + e * sum x: the first term is the fast kernels' (per chunk), the
 // second a row sum of the chunk (one MFMA against a fragment of ones) times e. Without a bias
