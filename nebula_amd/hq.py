@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from pathlib import Path
 from typing import Optional, Sequence
 
@@ -201,21 +202,50 @@ def convert_tq1_0(blocks: np.ndarray, K: int, N: int) -> tuple[np.ndarray, np.nd
 
 
 # ---------------------------------------------------------------- device calls
-def _stream_ptr(stream) -> Optional[int]:
-    import torch
+# The host side of a small call costs more than its kernel (4096 x 4096, M = 1: 4.8 us on the GPU):
+# the wrappers check a call's tensors in one expression each (the checks that name the fault run
+# only when it fails), take the stream's handle without building a stream object, and hand the
+# segments over as one packed buffer. One gemm call: 11.8 -> 7.1 us; a fused
+# call of three: 20.2 -> 12.0 (4.2 us of either in the C call, 1.4 in each output's allocation).
+class _Torch:
+    """torch, and what the wrappers need of it, loaded at the first device call."""
 
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    __slots__ = ("dtypes", "float32", "int8", "current_device", "raw_stream", "current_stream")
+
+    def __init__(self):
+        import torch
+
+        self.dtypes = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
+        self.float32, self.int8 = torch.float32, torch.int8
+        self.current_device = torch.cuda.current_device
+        self.raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        self.current_stream = torch.cuda.current_stream
+
+
+_torch: Optional[_Torch] = None
+
+
+def _load() -> _Torch:
+    global _torch
+    if _torch is None:
+        _torch = _Torch()
+    return _torch
+
+
+def _stream_ptr(stream) -> Optional[int]:
+    if stream is not None:
+        return stream.cuda_stream
+    t = _torch or _load()
+    if t.raw_stream is not None:
+        return t.raw_stream(t.current_device())
+    return t.current_stream().cuda_stream
 
 
 def _dt(t) -> int:
-    import torch
-
-    if t.dtype == torch.float16:
-        return DTYPE_F16
-    if t.dtype == torch.bfloat16:
-        return DTYPE_BF16
-    raise TypeError(f"activations must be float16 or bfloat16, got {t.dtype}")
+    code = (_torch or _load()).dtypes.get(t.dtype)
+    if code is None:
+        raise TypeError(f"activations must be float16 or bfloat16, got {t.dtype}")
+    return code
 
 
 def repack_device(fmt: int, linear, K: int, N: int, stream=None, bad_flag=None):
@@ -299,6 +329,28 @@ def _nbytes(t) -> int:
     return t.numel() * t.element_size()
 
 
+def _rows_ok(t, rows: int, cols: int, dtype) -> bool:
+    """Whether _check_rows accepts t."""
+    if t.dim() != 2 or t.dtype != dtype or not t.is_cuda:
+        return False
+    (r, c), (s0, s1) = t.shape, t.stride()
+    return r >= rows and c >= cols and (s1 == 1 or c <= 1) and (r <= 1 or s0 >= cols)
+
+
+def _weight_ok(fmt: int, Wp, scales, bias, K: int, N: int, group: int, dev: int) -> bool:
+    """Whether _check_weight accepts a weight for activations on GPU dev (int4 or ternary, K a
+    multiple of 128 and of group)."""
+    if not (Wp.is_cuda and scales.is_cuda and Wp.get_device() == dev and scales.get_device() == dev
+            and Wp.is_contiguous() and scales.is_contiguous() and group > 0 and not K % group and not K % 128):
+        return False
+    words = (N + 15) // 16 * (K // 128) * (256 if fmt == FORMAT_INT4 else 128)
+    n = K // group * N
+    if not (N > 0 and _nbytes(Wp) >= 4 * words and scales.element_size() == 2 and scales.numel() >= n):
+        return False
+    return bias is None or (fmt == FORMAT_INT4 and bias.is_cuda and bias.get_device() == dev and
+                            bias.dtype == (_torch or _load()).float32 and bias.is_contiguous() and bias.numel() >= n)
+
+
 def _check_rows(name: str, t, rows: int, cols: int, dtype) -> None:
     """t must be a device matrix of at least rows x cols elements of dtype, unit column stride."""
     if not t.is_cuda:
@@ -346,29 +398,34 @@ def gemm(fmt: int, X, Wp, scales, N: int, group: int = 128, out=None, stream=Non
     zero-filled before its first use; by default the library's own per-stream buffer is used.
     Shapes, dtypes, devices and strides are checked here: the kernels size their buffer
     descriptors from the shape, not from the allocations."""
-    import torch
-
     M, K = X.shape
-    _check_rows("X", X, M, K, X.dtype)
-    _dt(X)
-    _check_weight(fmt, Wp, scales, bias, K, N, group, X)
+    if not _rows_ok(X, M, K, X.dtype):
+        _check_rows("X", X, M, K, X.dtype)
+    dt = _dt(X)
+    if not (FORMAT_INT4 <= fmt <= FORMAT_TERNARY2 and _weight_ok(fmt, Wp, scales, bias, K, N, group, X.get_device())):
+        _check_weight(fmt, Wp, scales, bias, K, N, group, X)
     if out is None:
-        out = torch.empty((M, N), dtype=X.dtype, device=X.device)
-    _check_rows("out", out, M, N, X.dtype)
-    if out.device != X.device:
-        raise ValueError("out must be on X's device")
+        out = X.new_empty((M, N))
+        ldy = N
+    else:
+        if not _rows_ok(out, M, N, X.dtype):
+            _check_rows("out", out, M, N, X.dtype)
+        if out.device != X.device:
+            raise ValueError("out must be on X's device")
+        ldy = out.stride(0)
     wp, wb = _ws(workspace)
-    L = lib()
+    L = _lib or lib()
     if fmt == FORMAT_INT4:
-        st = L.hq_gemm_w4a16(X.data_ptr(), _dt(X), X.stride(0), Wp.data_ptr(), scales.data_ptr(),
-                             bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
+        st = L.hq_gemm_w4a16(X.data_ptr(), dt, X.stride(0), Wp.data_ptr(), scales.data_ptr(),
+                             bias.data_ptr() if bias is not None else None, out.data_ptr(), ldy,
                              M, K, N, group, wp, wb, _stream_ptr(stream))
     else:
         if bias is not None:
             raise ValueError("a bias is supported for int4 weights only")
-        st = L.hq_gemm_w2a16(X.data_ptr(), _dt(X), X.stride(0), Wp.data_ptr(), scales.data_ptr(), out.data_ptr(),
-                             out.stride(0), M, K, N, group, wp, wb, _stream_ptr(stream))
-    check(st)
+        st = L.hq_gemm_w2a16(X.data_ptr(), dt, X.stride(0), Wp.data_ptr(), scales.data_ptr(), out.data_ptr(),
+                             ldy, M, K, N, group, wp, wb, _stream_ptr(stream))
+    if st:
+        check(st)
     return out
 
 
@@ -377,35 +434,60 @@ def gemm_fused(fmt: int, X, segments: Sequence[tuple], group: int = 128, outs=No
     """segments: (Wp, scales, N) or (Wp, scales, N, bias) per projection; returns one output per
     segment. noalloc: run hq_gemm_fused_noalloc (its workspace is the library's static scratch;
     `outs` must then be given by a caller that cannot allocate)."""
-    import torch
-
     M, K = X.shape
-    _check_rows("X", X, M, K, X.dtype)
-    _dt(X)
-    if not 1 <= len(segments) <= MAX_SEGMENTS:
-        raise ValueError(f"need 1..{MAX_SEGMENTS} segments, got {len(segments)}")
-    if outs is None:
-        outs = [torch.empty((M, seg[2]), dtype=X.dtype, device=X.device) for seg in segments]
-    if len(outs) != len(segments):
+    if not _rows_ok(X, M, K, X.dtype):
+        _check_rows("X", X, M, K, X.dtype)
+    dt = _dt(X)
+    nseg = len(segments)
+    if not 1 <= nseg <= MAX_SEGMENTS:
+        raise ValueError(f"need 1..{MAX_SEGMENTS} segments, got {nseg}")
+    fresh = outs is None
+    if fresh:
+        outs = [X.new_empty((M, seg[2])) for seg in segments]
+    if len(outs) != nseg:
         raise ValueError("one output per segment")
-    arr = (Segment * len(segments))()
+    dev = X.get_device()
+    known = FORMAT_INT4 <= fmt <= FORMAT_TERNARY2
+    packed = bytearray(nseg * _SEGMENT.size)
     for i, (seg, y) in enumerate(zip(segments, outs)):
         wp, sc, n = seg[:3]
         b = seg[3] if len(seg) > 3 else None
-        _check_weight(fmt, wp, sc, b, K, n, group, X)
-        _check_rows(f"outs[{i}]", y, M, n, X.dtype)
-        arr[i] = Segment(wp.data_ptr(), sc.data_ptr(), b.data_ptr() if b is not None else None, y.data_ptr(),
-                         y.stride(0), n)
+        if not (known and _weight_ok(fmt, wp, sc, b, K, n, group, dev)):
+            _check_weight(fmt, wp, sc, b, K, n, group, X)
+        if not (fresh or _rows_ok(y, M, n, X.dtype)):
+            _check_rows(f"outs[{i}]", y, M, n, X.dtype)
+        _SEGMENT.pack_into(packed, i * _SEGMENT.size, wp.data_ptr(), sc.data_ptr(), b.data_ptr() if b is not None else 0,
+                           y.data_ptr(), n if fresh else y.stride(0), n)
+    arr = bytes(packed)
     if noalloc:
         if workspace is not None:
             raise ValueError("noalloc calls use the library's static scratch, not a workspace")
-        check(lib().hq_gemm_fused_noalloc(X.data_ptr(), _dt(X), X.stride(0), fmt, arr, len(segments), M, K, group,
-                                          _stream_ptr(stream)))
+        check((_fused_noalloc or _fused_calls()[1])(X.data_ptr(), dt, X.stride(0), fmt, arr, nseg, M, K, group,
+                                                    _stream_ptr(stream)))
         return outs
     wp, wb = _ws(workspace)
-    check(lib().hq_gemm_fused(X.data_ptr(), _dt(X), X.stride(0), fmt, arr, len(segments), M, K, group, wp, wb,
-                              _stream_ptr(stream)))
+    st = (_fused or _fused_calls()[0])(X.data_ptr(), dt, X.stride(0), fmt, arr, nseg, M, K, group, wp, wb,
+                                       _stream_ptr(stream))
+    if st:
+        check(st)
     return outs
+
+
+# hq_segment as bytes (the layout of Segment), and the fused entry points taking such a buffer.
+_SEGMENT = struct.Struct("@PPPPqI4x")
+assert _SEGMENT.size == ctypes.sizeof(Segment)
+_fused = _fused_noalloc = None
+
+
+def _fused_calls():
+    global _fused, _fused_noalloc
+    L = lib()
+    f, g = L["hq_gemm_fused"], L["hq_gemm_fused_noalloc"]  # indexing: function objects of their own
+    for own, public in ((f, L.hq_gemm_fused), (g, L.hq_gemm_fused_noalloc)):
+        own.restype = public.restype
+        own.argtypes = [ctypes.c_char_p if t is public.argtypes[4] else t for t in public.argtypes]
+    _fused, _fused_noalloc = f, g
+    return f, g
 
 
 # ---------------------------------------------------------------- the int8 path
@@ -438,18 +520,19 @@ def workspace_bytes_w8a8(M: int, K: int, N: int) -> int:
 def gemm_w8a8(X, Wp, scales, N: int, out=None, stream=None, workspace=None):
     """The int8 path: Y[M, N] (fp32) = scales[n] * sum_k int8(clamp(127 X)) W / 127, X fp32 [M, K]
     (M <= 16), Wp the int8 tile layout (repack_int8) on X's device, scales fp32 [N]."""
-    import torch
-
+    t = _torch or _load()
     M, K = X.shape
-    _check_rows("X", X, M, K, torch.float32)
+    if not _rows_ok(X, M, K, t.float32):
+        _check_rows("X", X, M, K, t.float32)
     if X.stride(0) % 4:
         raise ValueError("X's row stride must be a multiple of 4 elements")
-    for name, t, dt, n in (("Wp", Wp, torch.int8, lib().hq_int8_packed_bytes(K, N)), ("scales", scales, torch.float32, N)):
-        if t.device != X.device or t.dtype != dt or not t.is_contiguous() or t.numel() < n:
+    for name, v, dt, n in (("Wp", Wp, t.int8, (N + 15) // 16 * 16 * K if K % 128 == 0 else 0), ("scales", scales, t.float32, N)):
+        if v.device != X.device or v.dtype != dt or not v.is_contiguous() or v.numel() < n:
             raise ValueError(f"{name} must be a contiguous {dt} device tensor of at least {n} elements on X's device")
     if out is None:
-        out = torch.empty((M, N), dtype=torch.float32, device=X.device)
-    _check_rows("out", out, M, N, torch.float32)
+        out = X.new_empty((M, N))
+    elif not _rows_ok(out, M, N, t.float32):
+        _check_rows("out", out, M, N, t.float32)
     wp, wb = _ws(workspace)
     check(lib().hq_gemm_w8a8(X.data_ptr(), X.stride(0), Wp.data_ptr(), scales.data_ptr(), out.data_ptr(), out.stride(0),
                              M, K, N, wp, wb, _stream_ptr(stream)))
