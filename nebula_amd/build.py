@@ -23,7 +23,7 @@ BENCH_TOOL = BINDIR / "hq_bench_qgemm"
 STREAM_TOOL = BINDIR / "hq_stream_ceiling"
 ORACLE_DIR = ROOT / "oracle"
 
-SOURCES = ["hq_api.cpp", "hq_gguf.cpp", "hq_decode.hip", "hq_decode_ls.hip", "hq_prefill.hip", "hq_repack.hip", "hq_int8.hip"]
+SOURCES = ["hq_api.cpp", "hq_gguf.cpp", "hq_decode.hip", "hq_decode_ls.hip", "hq_rows.hip", "hq_prefill.hip", "hq_repack.hip", "hq_int8.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 

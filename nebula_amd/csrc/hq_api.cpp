@@ -143,15 +143,15 @@ hq_status get_internal_ws(hipStream_t stream, size_t need, void** out) {
 // small and the per-wavefront kernel (hq_decode.hip) is as fast or faster (M = 4, same-run
 // order-swapped timings on MI355X: 5120 x 5120 7.7 against 8.1 us, 5120 x 27648 15.9 against
 // 16.15 us, 27648 x 5120 even); from five rows on, the lockstep kernel (hq_decode_ls.hip),
-// which fetches each activation k-block once per workgroup, is, and above 16 rows only the
-// lockstep kernel takes them. With ternary weights the lockstep kernel's
+// which fetches each activation k-block once per workgroup, is, and above 16 rows it takes what
+// the shared row tiles (hq_rows.hip) do not. With ternary weights the lockstep kernel's
 // four-k-group configuration is faster from one row on (5120 x 27648 at M = 1: 12.8 us
 // against 14.7 us), so it is taken whenever the lockstep planner picks it. The general
 // kernels (bias, groups that are not multiples of 128) exist in the lockstep and (int4) the
 // X-resident family only.
 // HQ_DECODE_KERNEL=0 / 1 forces one of them for M <= 16 (tuning and tests).
 bool use_lockstep(int fmt, const hq::GemmDesc& d) {
-  if (d.M > 16 || d.gen) return true;  // only the lockstep kernel takes several row tiles
+  if (d.M > 16 || d.gen) return true;  // several row tiles (those hq_rows.hip does not take)
   const char* v = std::getenv("HQ_DECODE_KERNEL");
   if (v && *v) return std::atoi(v) != 0;
   if (d.M >= 5) return true;
@@ -281,13 +281,14 @@ hq::GemmDesc make_desc(uint32_t M, uint32_t K, uint32_t group, const uint32_t* N
 }
 
 // What a call runs: the kernel family, its tiling and the workspace it needs.
-enum class Kind { kDecode, kLockstep, kPrefill, kResident };
+enum class Kind { kDecode, kLockstep, kPrefill, kResident, kRows };
 struct Plan {
   Kind kind;
   hq::XrConfig xc{};
   hq::DecodeConfig c{};
   hq::LsConfig lc{};
   hq::PrefillConfig pc{};
+  hq::RowsConfig rc{};
   size_t need = 0;
 };
 
@@ -305,6 +306,12 @@ Plan make_plan(int fmt, const hq::GemmDesc& d, size_t cap = SIZE_MAX, int dtype 
   if (use_resident(fmt, d, cap, &p.xc)) {
     p.kind = Kind::kResident;
     p.need = hq::decode_xr_workspace_bytes(d, p.xc);
+    return p;
+  }
+  p.rc = hq::choose_rows(fmt, d, cap);
+  if (p.rc.ok) {
+    p.kind = Kind::kRows;
+    p.need = hq::rows_workspace_bytes(d, p.rc);
     return p;
   }
   if (!use_lockstep(fmt, d)) {
@@ -415,6 +422,7 @@ hq_status launch_plan(int fmt, int dtype, const hq::GemmDesc& d, const Plan& p, 
     case Kind::kLockstep:
       return from_hip(hq::launch_decode_ls(fmt, dtype, d, p.lc, w, fault, ls_spin(), s), "decode launch");
     case Kind::kResident: return from_hip(hq::launch_decode_xr(fmt, dtype, d, p.xc, w, s), "decode launch");
+    case Kind::kRows: return from_hip(hq::launch_rows(fmt, dtype, d, p.rc, w, s), "decode launch");
     case Kind::kDecode: break;
   }
   return from_hip(hq::launch_decode(fmt, dtype, d, p.c, w, s), "decode launch");
@@ -514,6 +522,9 @@ std::string describe(int fmt, int dtype, const hq::GemmDesc& d, const Plan& p) {
     std::snprintf(b, sizeof b, "hq_decode_kernel<%s,%s,T=%d,U=%d> workgroups=%d x %d wavefronts%s%s ws=%zu",
                   fmt_name(fmt), dt_name(dtype), p.c.T, decode_ring(p.c.T, p.c.U), p.c.SK, p.c.WK,
                   p.c.G ? " variable-width slabs" : "", p.need ? " cut slabs (fix-up)" : "", p.need);
+  } else if (p.kind == Kind::kRows) {
+    std::snprintf(b, sizeof b, "hq_rows_kernel<%s,%s,MT=%u> grid=%d pieces x slabs of 4 tiles, 8 wavefronts ws=%zu",
+                  fmt_name(fmt), dt_name(dtype), (d.M + 15u) / 16u, p.rc.S, p.need);
   } else if (p.kind == Kind::kLockstep) {
     std::snprintf(b, sizeof b,
                   "hq_decode_ls_kernel<%s,%s,KG=%d,GW=%d,T=%d,U=%d,MT=%d%s> grid=%d pieces x slabs of %d tiles, "

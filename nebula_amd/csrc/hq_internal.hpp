@@ -140,6 +140,15 @@ size_t decode_ls_workspace_bytes(const GemmDesc& d, const LsConfig& c);
 hipError_t launch_decode_ls(int fmt, int dtype, GemmDesc d, const LsConfig& c, void* ws, uint32_t* fault,
                             uint32_t spin, hipStream_t stream);
 
+// Shared row tiles (hq_rows.hip, 17 <= M <= 80): slabs of four column tiles, S pieces along K.
+struct RowsConfig {
+  int S;
+  bool ok;  // the kernel takes the call
+};
+RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MAX);
+size_t rows_workspace_bytes(const GemmDesc& d, const RowsConfig& c);
+hipError_t launch_rows(int fmt, int dtype, const GemmDesc& d, const RowsConfig& c, void* ws, hipStream_t stream);
+
 // One prefill launch: (16 * RT * WM)-row x 256-column tiles over the columns of d; psk
 // stream-K workgroups share the last tiles - dp tiles along K, dp workgroups own one tile
 // each.
