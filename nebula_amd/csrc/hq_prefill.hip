@@ -1010,8 +1010,10 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, const PrefillLaunch& cur, Pr
     *out = make_whole(4, d.nkb <= 16u ? 2 : 4, 2, d);
     return true;
   }
-  // A long K stays split over workgroups (K = 27648, M = 512, N = 5120: 170 us against 186-199).
-  if (cur.psk != 0 && d.nkb > 64u) return false;
+  // A long K stays split over workgroups (K = 27648, M = 512, N = 5120: int4 170 us against 186-199), for
+  // ternary, whose split is cheaper, already past 40 k-blocks (6144 x 5120, M = 400: 40.3 against 43.8
+  // us; 4096 x 5120, M = 448 39.1 -> 30.9).
+  if (cur.psk != 0 && d.nkb > (int4 ? 64u : 40u)) return false;
   if (t64 <= 2u * cus) {
     *out = int4 && t128 <= cus ? make_whole(8, 2, 2, d) : make_whole(4, 2, 2, d);
     return true;

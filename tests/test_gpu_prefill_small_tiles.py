@@ -70,6 +70,7 @@ def test_fused_segments_and_strides(cuda, monkeypatch):
     (O.INT4, 192, 4096, 20480, 128, "64x128 tiles=480"),
     (O.INT4, 96, 4096, 1024, 128, "whole=0 stream-K"),          # 16 tiles: the K split over workgroups
     (O.TERNARY2, 256, 14336, 4096, 128, "whole=0 stream-K"),    # a long K
+    (O.TERNARY2, 400, 6144, 5120, 256, "whole=0 stream-K"),
     (O.INT4, 1024, 4096, 14336, 32, "general> launch 0: 128-row tiles=448"),
     (O.INT4, 512, 4096, 14336, 32, "general> launch 0: 128-row 128-column tiles=448"),
 ])
