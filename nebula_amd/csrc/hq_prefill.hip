@@ -332,7 +332,8 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
     // scale (and bias) of that column in chunk g4 of the k-block, row (4 kb + g4) / g32.
     const uint32_t srows = GEN ? 4u * nkb / d.g32 : nkb / d.gkb;
     const __amdgpu_buffer_rsrc_t srs = make_rsrc(sg.S, ((srows - 1u) * sg.lds + sg.N) * 2u);
-    const __amdgpu_buffer_rsrc_t brs = make_rsrc(sg.B, GEN && sg.B ? ((srows - 1u) * sg.lds + sg.N) * 4u : 0u);
+    constexpr bool kBias = GEN && FMT == HQ_FORMAT_INT4;  // ternary weights have no bias to load
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t brs = make_rsrc(sg.B, kBias && sg.B ? ((srows - 1u) * sg.lds + sg.N) * 4u : 0u);
     uint32_t soff[kTilesPerWave];
 #pragma unroll
     for (int t = 0; t < kTilesPerWave; ++t) soff[t] = min((ct0 + t) * 16u + c16, sg.N - 1u) * 2u;
@@ -341,7 +342,7 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
     // Column tiles past the segment have an empty descriptor and read zero.
     u4 wr[kRing][kTilesPerWave];
     uint32_t sr[kRing][kTilesPerWave];
-    uint32_t br[GEN ? kRing : 1][kTilesPerWave];
+    uint32_t br[kBias ? kRing : 1][kTilesPerWave];
     auto load_b = [&](int slot, uint32_t kb) {
       const uint32_t kc = min(kb, kz - 1u);
       const uint32_t so = kc / d.gkb * sg.lds * 2u;
@@ -356,13 +357,14 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
         }
         if constexpr (GEN) {
           sr[slot][t] = __builtin_amdgcn_raw_buffer_load_b16(srs, soff[t] + grow * sg.lds * 2u, 0, 0);
-          br[slot][t] = __builtin_amdgcn_raw_buffer_load_b32(brs, soff[t] * 2u + grow * sg.lds * 4u, 0, 0);
         } else {
           sr[slot][t] = __builtin_amdgcn_raw_buffer_load_b16(srs, soff[t], so, 0);
         }
+        if constexpr (kBias)
+          br[slot][t] = __builtin_amdgcn_raw_buffer_load_b32(brs, soff[t] * 2u + grow * sg.lds * 4u, 0, 0);
       }
     };
-    const bool has_bias = GEN && sg.B != nullptr;
+    const bool has_bias = kBias && sg.B != nullptr;
 
 #pragma unroll
     for (int r = 0; r < RT; ++r)
@@ -371,8 +373,10 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
 
     // One k-block. Issue order per step: A(kb + 1) to LDS, then B(kb + kRing - 1) to
     // registers, so at the top of the next step vmcnt((kRing - 2) * kBLoads) leaves only the
-    // B loads of later k-blocks in flight (none with a ring of two).
-    constexpr int kBLoads = (GEN ? 3 : 2) * kTilesPerWave;  // weight, scale (and bias) loads per k-block
+    // B loads of later k-blocks in flight (none with a ring of two). The count holds only loads
+    // that the compiler keeps: one it can drop (its result unused) would let the wait pass before
+    // A(kb) has landed.
+    constexpr int kBLoads = (kBias ? 3 : 2) * kTilesPerWave;  // weight, scale (and bias) loads per k-block
     auto step = [&](uint32_t kb, int slot) {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm((kRing - 2) * kBLoads));  // A(kb), B(kb) landed for this wave
       kblock_barrier();  // ... for every wave (of the half); stage (kb+1)&1 is free
@@ -401,7 +405,7 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
           for (int t = 0; t < kTilesPerWave; ++t) {
             own[t] = sc[t];
             own_b[t] = 0u;
-            if constexpr (FMT == HQ_FORMAT_INT4) {
+            if constexpr (kBias) {
               const float s32 = f16_to_f32((uint16_t)sc[t]);
               if constexpr (DT == HQ_DTYPE_F16) {  // e = 8 s + b (0 without a bias), as fp16
                 if (has_bias)

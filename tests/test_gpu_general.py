@@ -173,3 +173,24 @@ def test_decode_27b_shape_bias(cuda):
     y = Dev(P).run()
     rows = np.arange(16)
     check(y, P, "K=5120 N=27648 M=16 bias", rows=rows)
+
+
+# Ternary weights have no bias loads: the 64-row x 256-column kernels (a ring of three k-blocks)
+# over seven and more k-blocks a piece, whole tiles and stream-K ranges that do not divide K.
+@pytest.mark.parametrize("xdt", [O.F16, O.BF16])
+@pytest.mark.parametrize("M,K,N,g,kv,plan", [
+    (300, 1152, 600, 32, dict(HQ_PREFILL_SK=0, HQ_PREFILL_RT=4), "64-row tiles=15 whole=15 stream-K workgroups=0"),
+    (300, 384, 600, 96, {}, "64-row tiles=15 whole=15 stream-K workgroups=0"),
+    (96, 4096, 1024, 64, dict(HQ_PREFILL_PSK=24), "64-row tiles=8 whole=0 stream-K workgroups=24"),
+    (256, 14336, 1024, 32, {}, "64-row tiles=16 whole=0 stream-K"),
+])
+def test_ternary_small_groups_in_64_row_tiles(cuda, xdt, M, K, N, g, kv, plan):
+    P = O.Problem(O.TERNARY2, M, K, N, g, xdt, seed=6900 + M)
+    D = Dev(P)
+    with env(**kv):
+        desc = hq.describe(O.TERNARY2, xdt, M, K, N, group=g)
+        assert ",general> launch 0: " + plan in desc, desc
+        y = D.run()
+        again = D.run()
+    assert bool((y == again).all())
+    check(y, P, f"ternary general 64-row tiles dt={xdt} M={M} K={K} g={g}")
