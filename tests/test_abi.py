@@ -201,21 +201,56 @@ def test_gemm_rejects_bad_arguments(kw, status):
 # Operands of 2 GiB or more: the kernels address every operand with 32-bit byte offsets, so
 # the entry points reject such shapes (HQ_ERR_SHAPE, no device work) instead of reading zeros
 # past the wrapped range.
-@pytest.mark.parametrize("kw,what", [
+RANGE_LIMITS = [
     (dict(M=16, ldx=1 << 26), "X spans"),                                  # 16 * 2^26 * 2 = 2 GiB
     (dict(M=16, ldy=1 << 26), "Y spans"),
     (dict(M=1, K=4096, N=1 << 26, ldy=1 << 26), "scales"),                 # 32 rows * 2^26 * 2 B
     (dict(M=1, K=1 << 16, ldx=1 << 16, N=1 << 16, ldy=1 << 16), "packed weights"),  # 2^12 tiles * 512 * 1 KiB
-])
+]
+
+
+@pytest.mark.parametrize("kw,what", RANGE_LIMITS)
 def test_gemm_rejects_operands_beyond_32_bit_offsets(kw, what):
     assert call_gemm(**kw) == hq.HQ_ERR_SHAPE
     assert what in hq.lib().hq_last_error().decode()
-    # One below each limit passes validation (and fails later only for the fake pointers).
+    # One below each limit is accepted. The calls must never launch (their pointers are made up, and
+    # a GPU may be visible), so a second segment whose scales are out of range ends them: the
+    # segments are checked in order, and the message names it.
+    wide = 1 << 26
     if what == "X spans":
-        assert call_gemm(M=16, ldx=(1 << 26) - 8) != hq.HQ_ERR_SHAPE
+        assert fused_with_a_bad_segment(hq.FORMAT_INT4, 16, 4096, (1 << 26) - 8, [4096, wide]) == hq.HQ_ERR_SHAPE
+        assert "segment 1" in hq.lib().hq_last_error().decode()
     if what == "packed weights":  # ternary packs half the bytes: the same shape is in range
-        assert call_gemm(fn="hq_gemm_w2a16", **kw) != hq.HQ_ERR_SHAPE
+        assert fused_with_a_bad_segment(hq.FORMAT_TERNARY2, 1, 1 << 16, 1 << 16, [1 << 16, wide]) == hq.HQ_ERR_SHAPE
+        assert "segment 1" in hq.lib().hq_last_error().decode()
         assert call_gemm(fn="hq_gemm_w2a16", M=1, K=1 << 16, ldx=1 << 16, N=1 << 17, ldy=1 << 17) == hq.HQ_ERR_SHAPE
+
+
+def fused_with_a_bad_segment(fmt, M, K, ldx, Ns):
+    segs = (hq.Segment * len(Ns))(*[hq.Segment(0x2000, 0x3000, None, 0x4000, n, n) for n in Ns])
+    return hq.lib().hq_gemm_fused(0x1000, hq.DTYPE_F16, ldx, fmt, segs, len(Ns), M, K, 128, None, 0, None)
+
+
+def test_no_call_with_made_up_pointers_launches(monkeypatch):
+    # What the range limits let through must end in another check: a call that passed every check
+    # here would launch on a visible GPU. HQ_OK and HQ_ERR_DEVICE are what a launch would return.
+    L, seen = hq.lib(), []
+
+    class Watch:
+        def __getattr__(self, name):
+            f = getattr(L, name)
+            if not name.startswith("hq_gemm"):
+                return f
+
+            def call(*a):
+                seen.append(f(*a))
+                return seen[-1]
+            return call
+
+    monkeypatch.setattr(hq, "_lib", Watch())
+    for kw, what in RANGE_LIMITS:
+        test_gemm_rejects_operands_beyond_32_bit_offsets(kw, what)
+    assert len(seen) >= 7 and not {hq.HQ_OK, hq.HQ_ERR_DEVICE} & set(seen)
 
 
 def test_range_limits_in_bias_fused_and_workspace_queries():
