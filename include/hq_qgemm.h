@@ -99,8 +99,11 @@ size_t hq_packed_words(hq_format fmt, uint32_t K, uint32_t N);
  * zero-filled by the caller before its first use (every call leaves it zero-filled
  * again). Calls sharing one workspace must not overlap in time (same stream, or ordered
  * by events), and a workspace shared by calls of several shapes needs the largest of their
- * sizes. The value is exactly what a one-projection call of this shape needs, with or
- * without a bias; for a fused call use hq_workspace_bytes_fused, which plans the call's own
+ * sizes. The value is exactly what a one-projection call of this shape asks for, with or
+ * without a bias: a call that writes partial sums rejects a smaller workspace. It can be more
+ * than the call writes, so that a size taken at many rows goes on serving fewer: up to 80 rows
+ * it does not fall as M grows through 17..80 (groups of 128) or 1..80 (int4 in groups of 32 or
+ * with a bias), whichever kernel takes which rows; for a fused call use hq_workspace_bytes_fused, which plans the call's own
  * segment list. Shapes whose operands would span 2 GiB or more (M * K * 2 bytes of X, the
  * scales, the packed weights) are rejected with HQ_ERR_SHAPE, as the GEMM calls reject them,
  * since the kernels address each operand with 32-bit offsets. Passing NULL instead

@@ -105,7 +105,9 @@ InternalWorkspace& internal_ws() {
   return *w;
 }
 
-hq_status get_internal_ws(hipStream_t stream, size_t need, void** out) {
+// use: what this call writes; need: what its shape asks for, so that a stream warmed up by a call
+// of many rows serves the calls of fewer rows that a capture then records.
+hq_status get_internal_ws(hipStream_t stream, size_t use, size_t need, void** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return fail(HQ_ERR_DEVICE, "hipGetDevice: %s", hipGetErrorString(e));
@@ -119,14 +121,25 @@ hq_status get_internal_ws(hipStream_t stream, size_t need, void** out) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   e = hipStreamIsCapturing(stream, &cap);
   if (e != hipSuccess) return fail(HQ_ERR_DEVICE, "hipStreamIsCapturing: %s", hipGetErrorString(e));
-  if (cap != hipStreamCaptureStatusNone)
+  if (cap != hipStreamCaptureStatusNone && slot.second < use)
     return fail(HQ_ERR_WORKSPACE,
                 "this shape needs %zu workspace bytes; pass a workspace (hq_workspace_bytes) or run "
                 "the shape once before capturing the stream",
-                need);
+                use);
+  if (cap != hipStreamCaptureStatusNone) {
+    *out = slot.first;
+    return HQ_OK;
+  }
   const size_t bytes = std::max(need, (size_t)1 << 20);
   void* p = nullptr;
-  if ((e = hipMalloc(&p, bytes)) != hipSuccess) return fail(HQ_ERR_DEVICE, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+  if ((e = hipMalloc(&p, bytes)) != hipSuccess) {
+    if (slot.second >= use) {  // the call itself can do without
+      (void)hipGetLastError();
+      *out = slot.first;
+      return HQ_OK;
+    }
+    return fail(HQ_ERR_DEVICE, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+  }
   if ((e = hipMemsetAsync(p, 0, bytes, stream)) != hipSuccess) {
     (void)hipFree(p);
     return fail(HQ_ERR_DEVICE, "hipMemsetAsync: %s", hipGetErrorString(e));
@@ -280,7 +293,13 @@ hq::GemmDesc make_desc(uint32_t M, uint32_t K, uint32_t group, const uint32_t* N
   return d;
 }
 
-// What a call runs: the kernel family, its tiling and the workspace it needs.
+// What a call runs: the kernel family, its tiling and the workspace it needs. `use` is what the plan
+// writes; `need`, what the call asks for, is more where a kernel that writes less (or nothing) has
+// taken a shape from one that cuts it along K: the shared row tiles and the general X-resident
+// kernel go on asking for the lockstep plan's pieces, prefill's whole 128-column tiles for the
+// stream-K plan's partial tiles. With the kernels' own needs alone, which jump to zero where such a
+// kernel takes over, a buffer sized at 80 rows (ternary 9984 x 10496: 0 bytes) failed at 33 (6.1 MB),
+// one sized at 1024 rows (3328 x 512) at every smaller M.
 enum class Kind { kDecode, kLockstep, kPrefill, kResident, kRows };
 struct Plan {
   Kind kind;
@@ -289,7 +308,7 @@ struct Plan {
   hq::LsConfig lc{};
   hq::PrefillConfig pc{};
   hq::RowsConfig rc{};
-  size_t need = 0;
+  size_t use = 0, need = 0;
 };
 
 // cap: the largest workspace the plan may use (the no-allocation entry point's scratch).
@@ -300,30 +319,34 @@ Plan make_plan(int fmt, const hq::GemmDesc& d, size_t cap = SIZE_MAX, int dtype 
   if (d.M > decode_max_m()) {
     p.kind = Kind::kPrefill;
     p.pc = hq::choose_prefill(fmt, d, cap, dtype);
-    p.need = hq::prefill_workspace_bytes(d, p.pc);
+    p.use = hq::prefill_workspace_bytes(d, p.pc);
+    p.need = std::max(p.use, p.pc.asked);
     return p;
   }
+  auto lockstep_need = [&] { return hq::decode_ls_workspace_bytes(d, hq::choose_decode_ls(fmt, d, cap, false)); };
   if (use_resident(fmt, d, cap, &p.xc)) {
     p.kind = Kind::kResident;
-    p.need = hq::decode_xr_workspace_bytes(d, p.xc);
+    p.use = p.need = hq::decode_xr_workspace_bytes(d, p.xc);
+    if (d.gen) p.need = std::max(p.use, lockstep_need());
     return p;
   }
   p.rc = hq::choose_rows(fmt, d, cap);
   if (p.rc.ok) {
     p.kind = Kind::kRows;
-    p.need = hq::rows_workspace_bytes(d, p.rc);
+    p.use = hq::rows_workspace_bytes(d, p.rc);
+    p.need = std::max(p.use, lockstep_need());
     return p;
   }
   if (!use_lockstep(fmt, d)) {
     p.kind = Kind::kDecode;
     p.c = hq::choose_decode(fmt, d);
-    p.need = hq::decode_workspace_bytes(d, p.c);
+    p.use = p.need = hq::decode_workspace_bytes(d, p.c);
     if (p.need <= cap) return p;
   }
   // The lockstep kernel takes every decode shape; under a cap with fewer pieces per slab.
   p.kind = Kind::kLockstep;
   p.lc = hq::choose_decode_ls(fmt, d, cap);
-  p.need = hq::decode_ls_workspace_bytes(d, p.lc);
+  p.use = p.need = hq::decode_ls_workspace_bytes(d, p.lc);
   return p;
 }
 
@@ -437,16 +460,16 @@ hq_status run_gemm(const void* X, hq_dtype dtype, int64_t ldx, hq_format fmt, co
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const Plan p = make_plan(fmt, d, SIZE_MAX, dtype);
   void* w = nullptr;
-  if (p.need > 0) {
-    if (ws) {
+  if (ws) {
+    if (p.use > 0) {  // a plan that writes nothing takes any workspace
       if (ws_bytes < p.need)
         return fail(HQ_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu this call needs", ws_bytes, p.need);
       if (reinterpret_cast<uintptr_t>(ws) % 256)
         return fail(HQ_ERR_ALIGNMENT, "workspace must be 256-byte aligned");
       w = ws;
-    } else if ((st = get_internal_ws(s, p.need, &w)) != HQ_OK) {
-      return st;
     }
+  } else if (p.need > 0 && (st = get_internal_ws(s, p.use, p.need, &w)) != HQ_OK) {
+    return st;
   }
   return launch_plan(fmt, dtype, d, p, w, fault_ptr(s), s);
 }
@@ -912,7 +935,7 @@ hq_status hq_gemm_w8a8(const float* X, int64_t ldx, const int8_t* Wp, const floa
       return fail(HQ_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu this call needs", ws_bytes, need);
     if (reinterpret_cast<uintptr_t>(ws) % 256) return fail(HQ_ERR_ALIGNMENT, "workspace must be 256-byte aligned");
     w = ws;
-  } else if ((st = get_internal_ws(s, need, &w)) != HQ_OK) {
+  } else if ((st = get_internal_ws(s, need, need, &w)) != HQ_OK) {
     return st;
   }
   return from_hip(hq::launch_w8a8(X, (uint32_t)ldx, Wp, scales, Y, (uint32_t)ldy, M, K, N, c, w, s), "int8 launch");
@@ -925,11 +948,11 @@ hq_status hq_gemm_fused_noalloc(const void* X, hq_dtype dtype, int64_t ldx, hq_f
   if (st != HQ_OK) return st;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const Plan p = make_plan(fmt, d, kScratchBytes, dtype);
-  if (p.need > kScratchBytes)
+  if (p.use > kScratchBytes)
     return fail(HQ_ERR_WORKSPACE, "this call needs %zu workspace bytes, more than the %zu-byte static scratch",
-                p.need, kScratchBytes);
+                p.use, kScratchBytes);
   void* w = nullptr;
-  if (p.need > 0 && (st = scratch_ptr(s, &w)) != HQ_OK) return st;
+  if (p.use > 0 && (st = scratch_ptr(s, &w)) != HQ_OK) return st;
   return launch_plan(fmt, dtype, d, p, w, fault_ptr_if_any(), s);
 }
 

@@ -965,17 +965,18 @@ hipError_t ls_launch_fd(const GemmDesc& d, const LsConfig& c, void* ws, uint32_t
 // Lockstep tiling: KG k-groups of four wavefronts, T tiles per wavefront (slabs of up to
 // 4 T tiles), ring depth U, and S pieces per slab chosen so that the grid covers the CUs.
 // HQ_DECODE_LS_KG / _T / _U / _S / _SW override (tuning and tests).
-LsConfig choose_decode_ls(int fmt, const GemmDesc& d, size_t ws_cap) {
+LsConfig choose_decode_ls(int fmt, const GemmDesc& d, size_t ws_cap, bool overrides) {
+  auto env = [&](const char* name, int dflt) { return overrides ? ls_env(name, dflt) : dflt; };
   const uint32_t cus = (uint32_t)cu_count();
   // Measured on MI355X (27B-class shapes, M = 4..16): two k-groups of four wavefronts,
   // two tiles per wavefront, two steps in flight; a K split only when the slabs alone
   // leave more than a quarter of the CUs idle.
   LsConfig c{2, 2, 1, 2, 4, 0, (int)std::min<uint32_t>(kLsMaxRowTiles, (d.M + 15u) / 16u)};
-  const int eKG = ls_env("HQ_DECODE_LS_KG", 0);
+  const int eKG = env("HQ_DECODE_LS_KG", 0);
   if (eKG == 1 || eKG == 2 || eKG == 4) c.KG = eKG;
-  const int eT = ls_env("HQ_DECODE_LS_T", 0);
+  const int eT = env("HQ_DECODE_LS_T", 0);
   if (eT == 1 || eT == 2 || eT == 4) c.T = eT;
-  const int eU = ls_env("HQ_DECODE_LS_U", 0);
+  const int eU = env("HQ_DECODE_LS_U", 0);
   if (eU >= 2 && eU <= 4) c.U = eU;
   // Snap to an instantiated (KG, T, U); several row tiles have two configurations (one or
   // two k-groups of four wavefronts, two tiles each, two steps in flight).
@@ -1032,7 +1033,7 @@ LsConfig choose_decode_ls(int fmt, const GemmDesc& d, size_t ws_cap) {
   // 1.25 slabs per CU (int4 5120 x 34816, M = 9..16: 25.3-27.2 -> 23.8-25.5 us; 4096 x 40960
   // 25.0-25.5 -> 21.7-22.1); ternary weights and 432 slabs measured slower, 544 even.
   // HQ_DECODE_LS_BAL = 0 / 1: off / on.
-  const int ebal = ls_env("HQ_DECODE_LS_BAL", -1);
+  const int ebal = env("HQ_DECODE_LS_BAL", -1);
   const bool one_tile = c.MT == 1 && c.GW == 4 && c.T == 2;
   const bool bal_fit = c.MT > 1 ? (4u * G <= 5u * cus || G > 2u * cus) : (fmt == HQ_FORMAT_INT4 && 4u * G <= 5u * cus);
   if ((c.MT > 1 || one_tile) && !d.gen && G > cus && G <= kMaxCounters && (ebal == 1 || (ebal != 0 && bal_fit))) {
@@ -1051,9 +1052,9 @@ LsConfig choose_decode_ls(int fmt, const GemmDesc& d, size_t ws_cap) {
     c.T = 2;
     c.U = 2;
   }
-  const int eSW = ls_env("HQ_DECODE_LS_SW", 0);
+  const int eSW = env("HQ_DECODE_LS_SW", 0);
   if (eSW >= 1 && eSW <= c.GW * c.T) c.SW = eSW;
-  const int eS = ls_env("HQ_DECODE_LS_S", 0);
+  const int eS = env("HQ_DECODE_LS_S", 0);
   if (eS >= 1) c.S = eS;
   c.S = std::max(1, std::min<int>({c.S, (int)d.nkb, (int)kMaxPieces}));
   if (c.S > 1 && ls_assign_slabs(x, (uint32_t)c.SW) > kMaxCounters) c.S = 1;

@@ -134,8 +134,9 @@ struct LsPlan {
 // Polls of the lockstep k-group barrier before it gives up (each poll sleeps ~64 cycles):
 // far beyond any correct launch, whose k-groups stay within one step of each other.
 constexpr uint32_t kLsSpinLimit = 1u << 22;
-// ws_cap: the largest workspace the plan may use (fewer pieces per slab below it).
-LsConfig choose_decode_ls(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MAX);
+// ws_cap: the largest workspace the plan may use (fewer pieces per slab below it). overrides: whether
+// the HQ_DECODE_LS_* variables are looked up.
+LsConfig choose_decode_ls(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MAX, bool overrides = true);
 size_t decode_ls_workspace_bytes(const GemmDesc& d, const LsConfig& c);
 hipError_t launch_decode_ls(int fmt, int dtype, GemmDesc d, const LsConfig& c, void* ws, uint32_t* fault,
                             uint32_t spin, hipStream_t stream);
@@ -167,6 +168,7 @@ struct PrefillLaunch {
 struct PrefillConfig {
   int n;
   PrefillLaunch l[2];
+  size_t asked;  // workspace of the plan that whole 128-column tiles took the place of (0: none did)
 };
 // ws_cap: the largest workspace the plan may use (fewer stream-K workgroups, or none, below it).
 // dtype: the activation type (the tile width depends on it; the workspace does not).

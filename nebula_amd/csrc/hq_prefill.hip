@@ -1068,6 +1068,7 @@ PrefillConfig choose_prefill(int fmt, const GemmDesc& d, size_t ws_cap, int dtyp
   if (c.n != 1) return c;
   PrefillLaunch small;
   if (choose_small_tiles(fmt, d, c.l[0], &small)) {
+    c.asked = prefill_workspace_bytes(d, c);
     c.l[0] = small;
     return c;
   }

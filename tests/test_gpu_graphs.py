@@ -65,6 +65,30 @@ def test_graph_replays_equal_eager(cuda, label, fmt, xdt, M, K, N, plan):
         assert bool(torch.equal(y1, y0)), f"{label}: eager call after replay {r} differs ({desc})"
 
 
+def test_capture_after_a_warm_up_of_more_rows(cuda):
+    # Ternary 9984 x 10496 runs whole slabs at 80 rows and K pieces at 33: the call of 80 rows leaves the
+    # stream's library workspace large enough for the other, which is then captured as it comes.
+    import torch
+
+    K, N = 9984, 10496
+    assert "hq_rows_kernel<ternary2,f16,MT=5> grid=1 pieces" in hq.describe(O.TERNARY2, O.F16, 80, K, N)
+    P = O.Problem(O.TERNARY2, 33, K, N, 128, O.F16, seed=9990)
+    D = DeviceProblem(P)
+    y0 = D.run()
+    side, out = torch.cuda.Stream(), torch.empty_like(y0)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        hq.gemm(O.TERNARY2, torch.zeros((80, K), dtype=torch.float16, device="cuda"), D.Wp, D.S, N, 128)
+    torch.cuda.synchronize()
+    g = capture(lambda: hq.gemm(O.TERNARY2, D.X, D.Wp, D.S, N, 128, out=out), side)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert bool(torch.equal(out, y0))
+        assert bool(torch.equal(D.run(), y0))
+
+
 def test_graph_replays_noalloc_fused(cuda):
     # The entry point that allocates nothing, captured: 27648 x 5120 at M = 16 (the lockstep
     # kernel's K pieces through the static scratch) in one fused call of two segments.
