@@ -1057,12 +1057,13 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, const PrefillLaunch& cur, Pr
 // Stream-K plans (short grids, long K) stay: 128-column tiles there were 1-40% slower.
 PrefillConfig choose_prefill(int fmt, const GemmDesc& d, size_t ws_cap, int dtype) {
   PrefillConfig c = choose_prefill_256(fmt, d, ws_cap);
-  if (const int f = env_int("HQ_PREFILL_TILE", 0)) {  // tuning / test override: RT * 100 + KS * 10 + TW
-    const PrefillLaunch l = make_whole(f / 100, f / 10 % 10, f % 10, d);
-    if (d.nkb >= (uint32_t)l.KS) {
-      c.n = 1;
-      c.l[0] = l;
-    }
+  // Tuning / test override: RT * 100 + KS * 10 + TW, one of the whole tiles launch_fd builds (822 for
+  // ternary weights only through this override: the planner gives those 422).
+  const int tile = env_int("HQ_PREFILL_TILE", 0);
+  const bool built = tile == 422 || tile == 442 || tile == 812 || tile == 814 || tile == 822 || (tile == 824 && !d.gen);
+  if (built && d.nkb >= (uint32_t)(tile / 10 % 10)) {
+    c.n = 1;
+    c.l[0] = make_whole(tile / 100, tile / 10 % 10, tile % 10, d);
     return c;
   }
   if (c.n != 1) return c;

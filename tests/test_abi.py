@@ -4,6 +4,8 @@ whose reference layout is bit-exact with the oracle's restatement of
 hydrogen/src/model/marlin_gemm.cu:446-455."""
 import ctypes
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -147,6 +149,26 @@ def test_describe_gemm_names_the_kernel_families(monkeypatch):
     assert "general" in hq.describe(hq.FORMAT_INT4, hq.DTYPE_BF16, 300, 4096, 4096, with_bias=True)
     with pytest.raises(hq.HQError):
         hq.describe(hq.FORMAT_TERNARY2, hq.DTYPE_F16, 4, 4096, 4096, with_bias=True)
+
+
+def test_prefill_tile_override_takes_only_tiles_that_are_built():
+    # Other values leave the planner's choice (in a process of its own: a height of 0 rows once ended
+    # it with a division by zero).
+    code = """
+import os
+from nebula_amd import hq
+plan = lambda **kw: [hq.describe(hq.FORMAT_INT4, hq.DTYPE_F16, 300, K, 4096, **kw) for K in (128, 4096)]
+plain, general = plan(), plan(group=32)
+for v in ("1", "9", "42", "99", "100", "400", "402", "420", "442000", "-442", "882", "x"):
+    os.environ["HQ_PREFILL_TILE"] = v
+    assert plan() == plain and plan(group=32) == general, v
+os.environ["HQ_PREFILL_TILE"] = "824"
+assert "128-row tiles=48 whole=48" in plan()[1] and plan(group=32) == general
+os.environ["HQ_PREFILL_TILE"] = "442"
+assert plan()[0] == plain[0] and "64x128 tiles=160" in plan()[1] and "64x128 tiles=160" in plan(group=32)[1]
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
 
 
 def test_device_status_without_faults():
