@@ -1159,11 +1159,9 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
   for (uint32_t i = 0; i < d.nseg; ++i) tiles += d.seg[i].ntiles;
   // The general kernels: two wavefronts per SIMD (their registers), no slab groups; not for the few
   // tiles whose slabs the lockstep kernel cuts along K (N = 256 and below: equal; N = 512, K = 4096:
-  // 7.3 -> 6.1 us here).
-  // Above eight rows a call of at most one tile per CU keeps the lockstep kernel's K pieces and with
-  // them the workspace such calls have always asked for, which grows with the row tiles (one-tile
-  // slabs here: 4096 x 4096 M = 16 9.7 -> 8.4 us, 4096 x 2048 8.9 -> 7.4).
-  if (d.gen && (8u * tiles < cus || (d.M > 8u && tiles <= cus))) return c;
+  // 7.3 -> 6.1 us here). Nine to 16 rows gain as much as fewer (M = 16, one-tile slabs: 1024 x 4096 7.8 ->
+  // 4.2, 4096 x 4096 9.0 -> 6.6, 5120 x 4096 10.3 -> 8.1, 14336 x 512 13.1 -> 9.3).
+  if (d.gen && 8u * tiles < cus) return c;
   auto waves_per_simd = [&](int T, int U) { return d.gen ? 2 : xr_waves_per_simd(fmt, T, U); };
   const int eT = env_int("HQ_XR_T", 0), eWK = env_int("HQ_XR_WK", 0), eU = env_int("HQ_XR_U", 0);
   const int eS = env_int("HQ_XR_S", 0), eG = env_int("HQ_XR_G", 0), eSG = env_int("HQ_XR_SG", 0);

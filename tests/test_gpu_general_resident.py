@@ -35,6 +35,19 @@ def test_default_plans(cuda, M, K, N):
     check(Dev(P).run(), P, f"general resident M={M} K={K} N={N}")
 
 
+# Nine to 16 rows over at most one tile per CU: one-tile slabs, ragged columns, an odd k-block count.
+@pytest.mark.parametrize("xdt", [O.F16, O.BF16])
+@pytest.mark.parametrize("M,K,N,g,bias", [(9, 1024, 4096, 32, "random"), (16, 2816, 1530, 64, None), (12, 4096, 4090, 32, "random"),
+                                          (16, 5120, 2048, 32, "random"), (13, 14336, 512, 32, "random")])
+def test_default_plans_of_nine_to_sixteen_rows(cuda, xdt, M, K, N, g, bias):
+    P = O.Problem(O.INT4, M, K, N, g, xdt, seed=9360 + M, bias=bias)
+    assert hq.describe(O.INT4, xdt, M, K, N, group=g, with_bias=bias is not None).startswith("hq_decode_xr_kernel<")
+    D = Dev(P)
+    y = D.run()
+    assert bool((y == D.run()).all())
+    check(y, P, f"general resident M={M} K={K} N={N} dt={xdt}")
+
+
 def test_segments_with_and_without_bias(cuda):
     import torch
 
