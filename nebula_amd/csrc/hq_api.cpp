@@ -298,7 +298,7 @@ hq::GemmDesc make_desc(uint32_t M, uint32_t K, uint32_t group, const uint32_t* N
 // taken a shape from one that cuts it along K: the shared row tiles and the general X-resident
 // kernel go on asking for the lockstep plan's pieces, prefill's whole 128-column tiles for the
 // stream-K plan's partial tiles. With the kernels' own needs alone, which jump to zero where such a
-// kernel takes over, a buffer sized at 80 rows (ternary 9984 x 10496: 0 bytes) failed at 33 (6.1 MB),
+// kernel takes over, a buffer sized at 80 rows (ternary 11264 x 11008: 0 bytes) failed at 33 (6.4 MB),
 // one sized at 1024 rows (3328 x 512) at every smaller M.
 enum class Kind { kDecode, kLockstep, kPrefill, kResident, kRows };
 struct Plan {

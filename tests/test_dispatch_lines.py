@@ -1,0 +1,29 @@
+"""CPU tests of where the planner's lines between kernels lie: shapes on both sides of each, measured on a
+256-CU device (without a GPU the planner assumes one), as the plan that was the faster there."""
+import pytest
+
+from nebula_amd import hq
+
+I4, T2, F16, BF16 = hq.FORMAT_INT4, hq.FORMAT_TERNARY2, hq.DTYPE_F16, hq.DTYPE_BF16
+
+
+def plan(fmt, dt, M, K, N, **kw):
+    import torch
+
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are those of a 256-CU device")
+    return hq.describe(fmt, dt, M, K, N, **kw)
+
+
+# Shared row tiles: slabs of four tiles that leave CUs idle lose over a long K, by rows.
+@pytest.mark.parametrize("fmt,M,slabs,kblocks,rows", [
+    (T2, 56, 130, 32, True), (T2, 56, 130, 48, False), (T2, 80, 130, 48, True), (T2, 80, 130, 96, False),
+    (I4, 64, 160, 152, False), (I4, 56, 136, 151, False), (I4, 80, 86, 128, False), (T2, 33, 86, 48, True),
+    (T2, 33, 86, 96, False), (T2, 20, 86, 32, True), (T2, 20, 86, 64, False),
+    (I4, 80, 172, 176, True), (T2, 56, 184, 128, True), (T2, 33, 172, 88, False),  # past one lockstep workgroup per CU
+    (T2, 20, 256, 32, True), (T2, 20, 256, 48, False), (T2, 33, 256, 64, True), (T2, 33, 256, 96, False),
+    (T2, 56, 256, 96, True), (I4, 80, 256, 112, True), (I4, 80, 240, 176, False),
+    (I4, 80, 32, 216, True), (T2, 56, 16, 216, True),                              # few slabs in eight pieces
+])
+def test_row_tiles_by_piece_length(fmt, M, slabs, kblocks, rows):
+    assert plan(fmt, F16, M, 128 * kblocks, 64 * slabs).startswith("hq_rows_kernel<" if rows else "hq_decode_ls_kernel<")

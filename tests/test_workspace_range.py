@@ -45,10 +45,10 @@ def test_prefill_asks_for_what_the_256_column_plan_does(monkeypatch, fmt, K, Ns,
 
 
 def test_a_plan_that_writes_nothing_takes_any_workspace():
-    # Ternary 9984 x 10496 at 80 rows runs whole slabs: it asks for what 33 rows need, but does not refuse
+    # Ternary 11264 x 11008 at 80 rows runs whole slabs: it asks for what 33 rows need, but does not refuse
     # a smaller buffer. At 33 rows, pieces: one byte less is refused (before any launch).
     L = hq.lib()
-    K, N = 9984, 10496
+    K, N = 11264, 11008
     big, small = need(hq.FORMAT_TERNARY2, 80, K, [N]), need(hq.FORMAT_TERNARY2, 33, K, [N])
     assert big >= small > 0
     assert "hq_rows_kernel" in hq.describe(hq.FORMAT_TERNARY2, hq.DTYPE_F16, 80, K, N)
