@@ -980,7 +980,8 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
 // left CUs idle or split their tiles along K over workgroups, paying for partial tiles in
 // memory; a 64- or 128-row x 128-column tile per CU whose k-blocks are split between the
 // workgroup's own groups of wavefronts keeps every SIMD busy and adds the groups' sums in LDS.
-// The choice is the same for both activation types (the workspace queries do not know it).
+// What the call asks for does not depend on the choice, so it can look at the activation type (the
+// workspace queries do not know it).
 // Measured on MI355X (K = 4096, previous plan -> this one, int4 fp16 / int4 bf16 / ternary fp16):
 //  * 64 x 128 tiles at most one per CU, four groups: M = 128, N = 14336 (224 tiles) 49.8 -> 23.4 /
 //    52.2 -> 27.3 / 30.5 -> 21.1 us; M = 333, N = 4096 (192) 46.0 -> 20.3 / 46.6 -> 26.4 / 35.4 ->
@@ -988,7 +989,11 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
 //    alone, that of a K split over workgroups with the work, so the line rises with K: at 64
 //    k-blocks (K = 8192) 64 tiles 37.4 -> 33.0 but 32 tiles 26.3 -> 32.3; at 216 (K = 27648)
 //    int4 240 tiles 126 -> 114, 120 tiles 92 -> 97, ternary 240 109 -> 104, 120 68 -> 94; at 112
-//    (K = 14336) 128 tiles int4 70 -> 57, ternary 46 -> 52. Below
+//    (K = 14336) 128 tiles int4 70 -> 57, ternary 46 -> 52. Int4 with bf16, whose weights take more
+//    VALU in the half as high tiles, from more tiles on: at 28 k-blocks 72 tiles 21.9 -> 24.2, 80 14% faster; at
+//    64 80 tiles 42.3 -> 45.2, 88 7% faster; at 112 112 tiles 62.1 -> 74.4, 152 7% faster; at 216 160 tiles
+//    116 -> 138, 248 12% faster. Ternary past 64 k-blocks: at 80 96 tiles fp16 34.6 -> 39.0, bf16 38.5 -> 40.2, 104 6
+//    and 13% faster; at 88 fp16 124 tiles 40.1 -> 44.1, 136 2-17% faster. Below
 //    17 k-blocks two groups do (K = 1024, M = 384, N = 4096: 16.5 -> 8.9 us, four groups 9.7).
 //  * more 64 x 128 tiles, up to two per CU: int4 takes 128 x 128 tiles of two groups while those
 //    fit one per CU (M = 256, N = 14336: 45.8 -> 35.1 us; bf16 M = 333, N = 7168 48.7 -> 38.7,
@@ -999,7 +1004,7 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
 //    weights serve half the rows (K = 4096, group 32 with a bias: M = 1024, N = 14336 fp16 143 -> 114
 //    us, bf16 183 -> 129, 128 x 256; M = 512, N = 14336 76.0 -> 67.7, 96.5 -> 77.4, 128 x 128; M = 160,
 //    N = 27648 84.7 -> 62.3, 102.8 -> 72.9, 64 x 128).
-bool choose_small_tiles(int fmt, const GemmDesc& d, const PrefillLaunch& cur, PrefillLaunch* out) {
+bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaunch& cur, PrefillLaunch* out) {
   if (d.M <= 64u || d.nkb < 4u) return false;
   for (const char* e : {"HQ_PREFILL_RT", "HQ_PREFILL_WM", "HQ_PREFILL_KS", "HQ_PREFILL_PSK", "HQ_PREFILL_SK", "HQ_PREFILL_TW"})
     if (env_set(e)) return false;  // a forced plan stays
@@ -1010,6 +1015,9 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, const PrefillLaunch& cur, Pr
     // Tiles from which the whole tiles win, for 256 CUs.
     uint32_t from = d.nkb <= 16u ? 32u : int4 && d.nkb > 32u ? 80u : 64u;
     if (d.nkb > 64u) from += int4 ? (d.nkb - 64u) / 2u : (d.nkb - 64u) * 7u / 5u;
+    if (int4 && dtype == HQ_DTYPE_BF16 && d.nkb > 24u)
+      from = d.nkb <= 40u ? 80u : std::min(240u, 88u + (std::max(d.nkb, 64u) - 64u) * 5u / 4u);
+    if (!int4 && d.nkb > 64u) from = std::max(from, dtype == HQ_DTYPE_BF16 ? 100u : std::min(136u, 3u * d.nkb - 136u));
     if ((uint64_t)t64 * 256u < (uint64_t)from * cus) return false;
     *out = make_whole(4, d.nkb <= 16u ? 2 : 4, 2, d);
     return true;
@@ -1068,7 +1076,7 @@ PrefillConfig choose_prefill(int fmt, const GemmDesc& d, size_t ws_cap, int dtyp
   }
   if (c.n != 1) return c;
   PrefillLaunch small;
-  if (choose_small_tiles(fmt, d, c.l[0], &small)) {
+  if (choose_small_tiles(fmt, d, dtype, c.l[0], &small)) {
     c.asked = prefill_workspace_bytes(d, c);
     c.l[0] = small;
     return c;

@@ -27,3 +27,16 @@ def plan(fmt, dt, M, K, N, **kw):
 ])
 def test_row_tiles_by_piece_length(fmt, M, slabs, kblocks, rows):
     assert plan(fmt, F16, M, 128 * kblocks, 64 * slabs).startswith("hq_rows_kernel<" if rows else "hq_decode_ls_kernel<")
+
+
+# Whole 64 x 128 prefill tiles against the K split over workgroups: from how many tiles, by K and type.
+@pytest.mark.parametrize("fmt,dt,M,kblocks,N,whole", [
+    (I4, BF16, 96, 28, 4608, False), (I4, F16, 96, 28, 4608, True), (I4, BF16, 128, 28, 5120, True),
+    (I4, BF16, 96, 64, 5120, False), (I4, F16, 96, 64, 5120, True), (I4, BF16, 96, 64, 6144, True),
+    (I4, BF16, 226, 98, 3456, False), (I4, BF16, 81, 112, 7168, False), (I4, F16, 81, 112, 7168, True),
+    (I4, BF16, 300, 216, 4096, False), (I4, BF16, 1024, 216, 1984, True),
+    (T2, F16, 226, 80, 3072, False), (T2, BF16, 192, 80, 4096, False), (T2, F16, 128, 80, 6656, True),
+    (T2, F16, 96, 88, 7936, False), (T2, F16, 333, 98, 2688, False), (T2, BF16, 333, 98, 2688, True), (T2, F16, 300, 64, 2048, True),
+])
+def test_small_prefill_tiles_by_type(fmt, dt, M, kblocks, N, whole):
+    assert ("64x128 tiles=" if whole else "whole=0 stream-K") in plan(fmt, dt, M, 128 * kblocks, N)
