@@ -1241,8 +1241,10 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
       // 4-tile slabs up to one and a half rounds beat 8-tile slabs of four wavefronts in one
       // round. Measured on MI355X (M = 1..8): ternary 5120 x 34816 20.0 -> 16.0 us at M = 1,
       // int4 4096 x 40960 22.8 -> 17.4 us; at 1.7 rounds (5120 x 55296) 8-tile slabs stay
-      // ahead from M = 4.
-      const bool t4_spill = t == 4 && 2u * wgs <= 3u * cus * per_cu;
+      // ahead from M = 4. The general kernels stop short of that: there the lockstep kernel's slabs
+      // of eight tiles cover three quarters of the CUs and run whole (1024 x 24576 M = 16 9.2 against
+      // 12.2 us, 3072 x 24576 18.6 against 20.4; at 368 slabs here 12-22% faster).
+      const bool t4_spill = t == 4 && (d.gen ? 2u * wgs < 3u * cus * per_cu : 2u * wgs <= 3u * cus * per_cu);
       if (per_cu < 1 || (wgs > cus * per_cu && !t4_spill)) continue;
       // Whole slabs leaving more than half of the CUs idle: try a split first.
       if (s == 1 && wgs * 2u < cus && total_slabs(d, t) * 2u <= cus * per_cu && d.nkb >= 2 && d.M <= 4u) break;
@@ -1265,6 +1267,17 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
       one_round = wgs <= cus * per_cu;
       break;
     }
+  }
+  // General kernels, whole slabs on at most two thirds of the CUs over a long K: the lockstep kernel,
+  // where its K pieces fill the CUs in one round. Lockstep -> here, bf16: 14336 x 10240 (160 slabs) M = 4 29.1 -> 30.1 us,
+  // 152 k-blocks 37.6 -> 40.1, 64 4% faster; 2-tile slabs 14336 x 4400 (seven pieces there) 16.4 -> 17.9, 88
+  // k-blocks even; 19456 x 5120 (six) 22.3 -> 22.9, 112 3-7% faster.
+  if (!forced && found && d.gen && c.S == 1 && (c.T == 2 || c.T == 4) && 3u * total_slabs(d, c.T) <= 2u * cus) {
+    uint32_t ls_slabs = 0;
+    for (uint32_t i = 0; i < d.nseg; ++i) ls_slabs += (d.seg[i].ntiles + 7u) / 8u;
+    const uint32_t pieces = (uint32_t)choose_decode_ls(fmt, d, ws_cap, false).S;
+    if (ls_slabs * pieces <= cus && 16u * ls_slabs * pieces >= 15u * cus &&
+        d.nkb >= (c.T == 4 ? 88u : pieces >= 7u ? 104u : 144u)) return c;
   }
   // General kernels, more 4-tile slabs than one round takes: two workgroups of four wavefronts per
   // CU, in as many rounds as it needs, where the rows fit twice (5120 x 27648, M = 4: 30.4 -> 25.4

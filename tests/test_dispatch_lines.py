@@ -40,3 +40,18 @@ def test_row_tiles_by_piece_length(fmt, M, slabs, kblocks, rows):
 ])
 def test_small_prefill_tiles_by_type(fmt, dt, M, kblocks, N, whole):
     assert ("64x128 tiles=" if whole else "whole=0 stream-K") in plan(fmt, dt, M, 128 * kblocks, N)
+
+
+# General int4 decode (group 32 with a bias): slabs that leave CUs idle, or need a second round, against
+# the lockstep kernel's.
+@pytest.mark.parametrize("M,kblocks,N,resident", [
+    (16, 8, 24576, True), (16, 24, 24576, False), (9, 40, 24576, False), (16, 24, 23552, True), (4, 16, 24576, True),
+    (4, 112, 10240, False), (2, 152, 10240, False), (4, 64, 10240, True), (1, 112, 9216, True),
+    (4, 112, 4400, False), (1, 152, 4400, False), (4, 88, 4400, True), (6, 152, 4400, True),
+    (4, 152, 5120, False), (4, 112, 5120, True), (4, 112, 2560, True),
+])
+def test_general_resident_slabs(M, kblocks, N, resident):
+    d = plan(I4, BF16, M, 128 * kblocks, N, group=32, with_bias=True)
+    assert d.startswith("hq_decode_xr_kernel<" if resident else "hq_decode_ls_kernel<"), d
+    if (M, kblocks, N) == (16, 8, 24576):  # two workgroups of four wavefronts per CU
+        assert "x 4 wavefronts" in d
