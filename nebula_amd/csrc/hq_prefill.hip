@@ -993,7 +993,8 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
 //    VALU in the half as high tiles, from more tiles on: at 28 k-blocks 72 tiles 21.9 -> 24.2, 80 14% faster; at
 //    64 80 tiles 42.3 -> 45.2, 88 7% faster; at 112 112 tiles 62.1 -> 74.4, 152 7% faster; at 216 160 tiles
 //    116 -> 138, 248 12% faster. Ternary past 64 k-blocks: at 80 96 tiles fp16 34.6 -> 39.0, bf16 38.5 -> 40.2, 104 6
-//    and 13% faster; at 88 fp16 124 tiles 40.1 -> 44.1, 136 2-17% faster. Below
+//    and 13% faster; at 88 fp16 124 tiles 40.1 -> 44.1, 136 2-17% faster; in groups of 64 from a few more (at 150
+//    186 tiles 72.0 -> 76.4). Below
 //    17 k-blocks two groups do (K = 1024, M = 384, N = 4096: 16.5 -> 8.9 us, four groups 9.7).
 //  * more 64 x 128 tiles, up to two per CU: int4 takes 128 x 128 tiles of two groups while those
 //    fit one per CU (M = 256, N = 14336: 45.8 -> 35.1 us; bf16 M = 333, N = 7168 48.7 -> 38.7,
@@ -1003,7 +1004,11 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
 //    256 tiles (one group) by rounds, in place of 64-row tiles of 256 columns, whose dequantised
 //    weights serve half the rows (K = 4096, group 32 with a bias: M = 1024, N = 14336 fp16 143 -> 114
 //    us, bf16 183 -> 129, 128 x 256; M = 512, N = 14336 76.0 -> 67.7, 96.5 -> 77.4, 128 x 128; M = 160,
-//    N = 27648 84.7 -> 62.3, 102.8 -> 72.9, 64 x 128).
+//    N = 27648 84.7 -> 62.3, 102.8 -> 72.9, 64 x 128). The 64-row tiles stay where their own rounds (one tile
+//    per CU each) come out cheaper: those run three and four to a CU, and the ternary ones, whose weights
+//    take few instructions, lose little by serving half the rows. Group 64, 64-row tiles -> the cheapest of
+//    the others: ternary bf16 1920 x 23680 M = 643 (1023 tiles, four rounds) 66.7 -> 77.0 us, 2176 x 15337 M = 736
+//    (720) 70.3 -> 80.0, but 864 tiles 16% and 260-384 tiles 8-23% faster; int4 fp16 1023 tiles 80.4 -> 86.4.
 bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaunch& cur, PrefillLaunch* out) {
   if (d.M <= 64u || d.nkb < 4u) return false;
   for (const char* e : {"HQ_PREFILL_RT", "HQ_PREFILL_WM", "HQ_PREFILL_KS", "HQ_PREFILL_PSK", "HQ_PREFILL_SK", "HQ_PREFILL_TW"})
@@ -1018,6 +1023,7 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaun
     if (int4 && dtype == HQ_DTYPE_BF16 && d.nkb > 24u)
       from = d.nkb <= 40u ? 80u : std::min(240u, 88u + (std::max(d.nkb, 64u) - 64u) * 5u / 4u);
     if (!int4 && d.nkb > 64u) from = std::max(from, dtype == HQ_DTYPE_BF16 ? 100u : std::min(136u, 3u * d.nkb - 136u));
+    if (!int4 && d.gen && d.nkb > 64u) from = std::max(136u, from * 9u / 8u);
     if ((uint64_t)t64 * 256u < (uint64_t)from * cus) return false;
     *out = make_whole(4, d.nkb <= 16u ? 2 : 4, 2, d);
     return true;
@@ -1026,6 +1032,12 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaun
   // ternary, whose split is cheaper, already past 40 k-blocks (6144 x 5120, M = 400: 40.3 against 43.8
   // us; 4096 x 5120, M = 448 39.1 -> 30.9).
   if (cur.psk != 0 && d.nkb > (int4 ? 64u : 40u)) return false;
+  // So do three equal pieces, which leave no workgroup with a longer one, of ternary weights: group 64 from 30
+  // k-blocks (36, 260-340 tiles: 3-13% faster than 64 x 128 tiles, 35 and 37: 0-18% slower), fp16 in multiples of
+  // 128 from 36 while the tiles are few (280 tiles 34.3 against 36.1 us; bf16 there 11-22% slower).
+  if (!int4 && cur.psk == 3u * cur.tiles && d.nkb % 3u == 0u &&
+      (d.gen ? d.nkb >= 30u : dtype == HQ_DTYPE_F16 && d.nkb >= 36u && 17u * cus >= 15u * t64))
+    return false;
   if (t64 <= 2u * cus) {
     *out = int4 && t128 <= cus ? make_whole(8, 2, 2, d) : make_whole(4, 2, 2, d);
     return true;
@@ -1038,6 +1050,9 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaun
     return (double)(t / (2u * cus)) + (rest == 0u ? 0.0 : rest <= cus ? 0.6 : 0.95);
   };
   const double c422 = 41.0 * rounds(t64), c812 = 71.5 * rounds(t128), c814 = 119.0 * rounds(make_launch(8, 1, d).tiles);
+  const bool bf16 = dtype == HQ_DTYPE_BF16;
+  const double round64 = int4 ? (bf16 ? 48.0 : 38.5) : (bf16 ? 35.5 : 38.0);
+  if (cur.psk == 0 && round64 * ((cur.tiles + cus - 1u) / cus) < std::min({c422, c812, c814})) return false;
   *out = c814 <= c422 && c814 <= c812 ? make_whole(8, 1, 4, d) : c812 <= c422 ? make_whole(8, 1, 2, d) : make_whole(4, 2, 2, d);
   return true;
 }

@@ -42,6 +42,18 @@ def test_small_prefill_tiles_by_type(fmt, dt, M, kblocks, N, whole):
     assert ("64x128 tiles=" if whole else "whole=0 stream-K") in plan(fmt, dt, M, 128 * kblocks, N)
 
 
+# Ternary prefill in groups of 64 past one 64 x 128 tile per CU: the 64-row tiles stay where their rounds of
+# one tile per CU are cheaper, the K split over a long K.
+@pytest.mark.parametrize("dt,group,M,kblocks,N,tile", [
+    (BF16, 64, 643, 15, 23680, "64-row tiles=1023 whole"), (BF16, 64, 736, 17, 15360, "64-row tiles=720 whole"),
+    (F16, 64, 736, 17, 15360, "128-row tiles=360"), (BF16, 64, 891, 46, 15360, "128-row tiles=420"),
+    (F16, 64, 144, 150, 7936, "whole=0 stream-K"), (BF16, 64, 300, 27, 7168, "64x128"),
+])
+def test_ternary_tiles_past_one_per_cu(dt, group, M, kblocks, N, tile):
+    d = plan(T2, dt, M, 128 * kblocks, N, group=group)
+    assert tile in d, d
+
+
 # General int4 decode (group 32 with a bias): slabs that leave CUs idle, or need a second round, against
 # the lockstep kernel's.
 @pytest.mark.parametrize("M,kblocks,N,resident", [

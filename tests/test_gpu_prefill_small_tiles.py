@@ -81,3 +81,19 @@ def test_default_plans(cuda, fmt, M, K, N, g, want):
         pytest.skip("the boundaries are those of a 256-CU device")
     for dt in (O.F16, O.BF16):
         assert want in hq.describe(fmt, dt, M, K, N, group=g)
+
+
+# Three equal pieces along K (the planner needs the device's occupancy for them): ternary fp16, and both
+# types in groups of 64, stay split; pieces that do not come out equal take the whole tiles.
+@pytest.mark.parametrize("dt,group,M,kblocks,N,split", [
+    (O.F16, 128, 300, 36, 7168, True), (O.BF16, 128, 300, 36, 7168, False), (O.F16, 128, 300, 35, 7168, False),
+    (O.F16, 128, 300, 36, 8704, False), (O.F16, 64, 167, 36, 14336, True), (O.BF16, 64, 1762, 39, 1280, True),
+    (O.BF16, 64, 167, 37, 14336, False), (O.BF16, 64, 300, 27, 7168, False),
+])
+def test_three_equal_pieces_stay_split(cuda, dt, group, M, kblocks, N, split):
+    import torch
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the boundaries are those of a 256-CU device")
+    d = hq.describe(O.TERNARY2, dt, M, 128 * kblocks, N, group=group)
+    assert ("whole=0 stream-K" if split else "64x128 tiles=") in d, d
