@@ -1,7 +1,7 @@
 """Failure reporting of kernels that give up a bounded wait, forced from the host.
 
-The lockstep decode kernel's k-group barrier and the barrier of the two K halves of a prefill
-tile (KS = 2) poll an LDS arrival count a bounded number of times. HQ_DECODE_LS_SPIN=0 makes
+The lockstep decode kernel's k-group barrier and the barrier of the two or four K groups of a
+prefill tile poll an LDS arrival count a bounded number of times. HQ_DECODE_LS_SPIN=0 makes
 every wait give up at once: the wavefronts carry on (so the kernel exits normally, with wrong
 outputs) and set the host-visible fault word, which the next hq_device_status() (or the next
 GEMM call) reports as HQ_ERR_DEVICE and clears.
@@ -53,14 +53,15 @@ def test_kgroup_barrier_timeout_is_reported(cuda):
     check(y, P.reference(), O.F16, "after a reported fault", P)
 
 
-def test_prefill_k_halves_barrier_timeout_is_reported(cuda):
-    # A prefill tile split in two K halves of one workgroup meets per k-block at an LDS
-    # arrival count; giving up is reported like the decode k-group barrier.
+@pytest.mark.parametrize("plan", [dict(KS=2, WM=1, SK=0, TAIL=0), dict(TILE=442)])
+def test_prefill_k_halves_barrier_timeout_is_reported(cuda, plan):
+    # A prefill tile split in two K halves, or four quarters, of one workgroup meets per k-block at an
+    # LDS arrival count; giving up is reported like the decode k-group barrier.
     from test_gpu_parity import check, prefill_env
 
     P = O.Problem(O.INT4, 300, 2048, 1000, 128, O.F16, seed=9110)
     D = DeviceProblem(P)
-    with prefill_env(KS=2, WM=1, SK=0, TAIL=0):
+    with prefill_env(**plan):
         assert "k-split in workgroup" in hq.describe(O.INT4, O.F16, 300, 2048, 1000)
         D.run()
         hq.device_status()  # no fault so far

@@ -97,3 +97,25 @@ def test_three_equal_pieces_stay_split(cuda, dt, group, M, kblocks, N, split):
         pytest.skip("the boundaries are those of a 256-CU device")
     d = hq.describe(O.TERNARY2, dt, M, 128 * kblocks, N, group=group)
     assert ("whole=0 stream-K" if split else "64x128 tiles=") in d, d
+
+
+# The plans of test_default_plans as they run, the new tiles at the sizes they serve: grids of 192 to 480 tiles over
+# several row bands, four groups over 32 and more k-blocks, the general 128-row tiles over more than one
+# round. Each row band's first and last row and a few between are compared.
+@pytest.mark.parametrize("fmt,xdt,M,K,N,group,bias", [
+    (O.INT4, O.F16, 128, 4096, 14336, 128, None), (O.INT4, O.BF16, 384, 1024, 4096, 128, None),
+    (O.INT4, O.BF16, 256, 4096, 14336, 128, None), (O.TERNARY2, O.F16, 256, 4096, 14336, 128, None),
+    (O.TERNARY2, O.BF16, 192, 6144, 20480, 256, None), (O.INT4, O.F16, 192, 4096, 20480, 128, None),
+    (O.INT4, O.F16, 1024, 4096, 14336, 32, "random"), (O.INT4, O.BF16, 1024, 4096, 14336, 32, "random"),
+    (O.INT4, O.F16, 512, 4096, 14336, 32, "random"), (O.INT4, O.BF16, 512, 4096, 14336, 64, "random"),
+    (O.INT4, O.F16, 600, 1024, 28000, 32, "random"),
+])
+def test_default_plans_compute(cuda, fmt, xdt, M, K, N, group, bias):
+    import numpy as np
+
+    d = hq.describe(fmt, xdt, M, K, N, group=group, with_bias=bias is not None)
+    assert "whole=0" not in d, d
+    P = O.Problem(fmt, M, K, N, group, xdt, seed=8700 + M, bias=bias)
+    rows = np.unique(np.concatenate([np.arange(0, M, 64), np.arange(63, M, 64), [M // 2 + 5, M - 1]]))
+    y = Dev(P).run(bias=bias is not None)
+    check_general(y, P, f"{d} M={M} K={K} N={N}", rows=rows)
