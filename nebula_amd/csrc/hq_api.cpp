@@ -393,11 +393,11 @@ bool take_fault() {
 hq_status fault_status() {
   return fail(HQ_ERR_DEVICE,
               "a launch gave up waiting at a k-group barrier (the lockstep decode kernel's k-groups, or the "
-              "two K halves of a prefill tile): the outputs of that launch are wrong (fault word reported by "
+              "K halves or quarters of a prefill tile): the outputs of that launch are wrong (fault word reported by "
               "the device)");
 }
 uint32_t ls_spin() {
-  // Polls of the kernels' bounded barriers (lockstep k-groups, prefill K halves); tests: a
+  // Polls of the kernels' bounded barriers (lockstep k-groups, prefill K groups); tests: a
   // small limit forces the fault path.
   const char* v = std::getenv("HQ_DECODE_LS_SPIN");
   return v && *v ? (uint32_t)std::strtoul(v, nullptr, 10) : hq::kLsSpinLimit;

@@ -150,7 +150,7 @@ RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MAX);
 size_t rows_workspace_bytes(const GemmDesc& d, const RowsConfig& c);
 hipError_t launch_rows(int fmt, int dtype, const GemmDesc& d, const RowsConfig& c, void* ws, hipStream_t stream);
 
-// One prefill launch: (16 * RT * WM)-row x 256-column tiles over the columns of d; psk
+// One prefill launch: (16 * RT * WM)-row x (64 * TW)-column tiles over the columns of d; psk
 // stream-K workgroups share the last tiles - dp tiles along K, dp workgroups own one tile
 // each.
 struct PrefillLaunch {
@@ -176,8 +176,8 @@ PrefillConfig choose_prefill(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MA
 // Workspace bytes of a prefill call (0 without stream-K): the counter area, then two fp32
 // partial tiles per stream-K workgroup.
 size_t prefill_workspace_bytes(const GemmDesc& d, const PrefillConfig& c);
-// Prefill (M > 16): MFMA tile kernel.
-// fault / spin: the fault word and the poll bound of the K halves' barrier (KS = 2 launches).
+// Prefill (M > 80): MFMA tile kernel.
+// fault / spin: the fault word and the poll bound of the K groups' barriers (KS = 2 and 4 launches).
 hipError_t launch_prefill(int fmt, int dtype, const PrefillConfig& c, void* ws, uint32_t* fault, uint32_t spin,
                           hipStream_t stream);
 

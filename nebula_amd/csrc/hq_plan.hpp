@@ -72,13 +72,13 @@ struct PrefillPlan {
   uint32_t xcd;     // 1: number the whole-tile workgroups XCD-major (dp % 8 == 0)
   uint32_t L, rem;  // stream-K ranges: begin(s) = s * L + min(s, rem)
   uint32_t nkb_m;   // plan_div_magic(nkb)
-  uint32_t nb;      // 256-column blocks over all segments (tile = row band * nb + block)
+  uint32_t nb;      // column blocks (256 columns, 128 with TW = 2) over all segments (tile = row band * nb + block)
   uint32_t bands;   // row bands (tiles = bands * nb)
   uint32_t gb;      // whole tiles are visited in groups of gb row bands, column-block major
   float* part;      // [psk][2][tile] fp32 partial tiles (null when psk == 0)
   uint32_t* cnt;    // [tiles - dp] arrival counters, zero between launches
   uint32_t* fault;  // host-visible word set to 1 when a bounded wait gives up (may be null)
-  uint32_t spin;    // polls before the K halves' k-block barrier gives up (KS = 2)
+  uint32_t spin;    // polls before a K group's k-block barrier gives up (KS = 2, 4)
 };
 
 // Exact u / d for any 32-bit u without a divide instruction: m = floor((2^32 - 1) / d)

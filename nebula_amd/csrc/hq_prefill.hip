@@ -42,7 +42,7 @@ constexpr int kValuPerFrag = 7;
 
 // Ternary weights with bf16 activations: t * s rounds to t times the bf16 rounding of the fp16
 // scale s (t is -1, 0 or 1), so a group has one bf16 pattern P to place under its signs.
-// Read as fp16, P is an ordinary number (the exponents of fp16 values in bf16, 103..142, give
+// Read as fp16, P is an ordinary number (the exponents of fp16 values in bf16, 103..143, give
 // fp16 exponent fields 12..17), so v_pk_mul_f16 of the fields' +-2.0 by "half of P" (P - 0x400:
 // one less in the exponent field) gives +-P exactly. Both halves of the result hold P - 0x400
 // (0 for a zero scale). Forming t * s in fp32 and rounding each weight took 28 VALU
@@ -168,9 +168,9 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
 
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t kh = KS > 1 ? wave_all / (4u * WM) : 0u;           // K half (KS = 2)
-  const uint32_t wave = KS > 1 ? wave_all % (4u * WM) : wave_all;    // wavefront within its half
-  char* const stages = smem + kh * 2u * kStageBytes;                 // this half's two LDS stages
+  const uint32_t kh = KS > 1 ? wave_all / (4u * WM) : 0u;           // K group
+  const uint32_t wave = KS > 1 ? wave_all % (4u * WM) : wave_all;    // wavefront within its K group
+  char* const stages = smem + kh * 2u * kStageBytes;                 // this K group's two LDS stages
   const uint32_t c16 = lane & 15u, g4 = lane >> 4;
   const uint32_t wm = wave / 4u, wn = wave % 4u;
   const uint32_t wrow0 = wm * 16u * RT;  // first tile row of this wavefront
@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(256 * WM * KS, WM == 1 && RT == 8 && KS == 1 ?
     constexpr int kBLoads = (kBias ? 3 : 2) * kTilesPerWave;  // weight, scale (and bias) loads per k-block
     auto step = [&](uint32_t kb, int slot) {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm((kRing - 2) * kBLoads));  // A(kb), B(kb) landed for this wave
-      kblock_barrier();  // ... for every wave (of the half); stage (kb+1)&1 is free
+      kblock_barrier();  // ... for every wave (of the K group); stage (kb+1)&1 is free
       load_a((kb + 1) & 1u, kb + 1);
       load_b((slot + kRing - 1) % kRing, kb + kRing - 1);
       // Keep this step's loads ahead of its compute: vmcnt retires in issue order, so a load
