@@ -1063,20 +1063,23 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaun
 // wavefronts of 32 columns, two workgroups per CU) in place of a one-round whole-tile grid
 // that leaves the CUs one workgroup each or uneven: at the same tile count as 64-row tiles
 // each dequantised weight serves twice the rows, and against a 128-row tile split in two K
-// halves the CU holds two independent tiles. The choice depends on the activation type (the
-// fp16 256-column kernel runs an explicit instruction order, the bf16 one forms its weights
-// in fp32) but not the workspace: every plan it swaps needs none. Measured on MI355X (best of
+// halves the CU holds two independent tiles. The choice depends on the activation type (int4
+// with bf16 forms its weights in fp32 and has no explicit instruction order at 256 columns; ternary
+// with bf16 has both as fp16 does, and still times like int4 there) but not the workspace: every
+// plan it swaps needs none. Measured on MI355X (best of
 // two alternated runs, K = 4096..5120, M = 81..1536):
 //  * in place of 64-row whole tiles (216-344): 8-18% faster for int4 fp16 (5120 x 7168
 //    M = 768 79.6 -> 68.9 us), 7-30% for bf16 (5120 x 34816 M = 96 104.6 -> 80.5 us), 5-11%
 //    for ternary fp16 where the 64-row tiles outnumber the CUs (216 tiles at 5120 x 27648:
 //    -4..+2%);
 //  * in place of the K split (192-256 tiles): fp16 3-6% faster (the fused QKV width at M =
-//    1024, int4: 72.8 -> 68.8 us), bf16 within -4..+2%;
+//    1024, int4: 72.8 -> 68.8 us; over K = 27648, 220 tiles, 3-4% slower), int4 bf16 within -7..+2%,
+//    ternary bf16 2-4% faster (over K = 27648 2% slower);
 //  * in place of 272-336 128-row whole tiles (544-672 128-column tiles): bf16 8-11% faster,
 //    also over a long K (27648 x 5120, 17408 x 5120, 16384 x 6144, 8192 x 8192 at M = 1152..
 //    2048: 8-13%), fp16 6-13% slower; bf16 at 408 (816) 8% slower, at 432-1728 (864-3456) up
-//    to 11% slower.
+//    to 11% slower. Ternary bf16 with the scale placed by one multiply: 264-344 tiles 8-11% faster (4096 x 11008
+//    M = 1024 102.6 -> 92.4 us; fp16 83.1 -> 91.8), 408 6% slower.
 // Stream-K plans (short grids, long K) stay: 128-column tiles there were 1-40% slower.
 PrefillConfig choose_prefill(int fmt, const GemmDesc& d, size_t ws_cap, int dtype) {
   PrefillConfig c = choose_prefill_256(fmt, d, ws_cap);
