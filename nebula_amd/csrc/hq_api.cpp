@@ -298,7 +298,7 @@ hq::GemmDesc make_desc(uint32_t M, uint32_t K, uint32_t group, const uint32_t* N
 // taken a shape from one that cuts it along K: the shared row tiles and the general X-resident
 // kernel go on asking for the lockstep plan's pieces, prefill's whole 128-column tiles for the
 // stream-K plan's partial tiles. With the kernels' own needs alone, which jump to zero where such a
-// kernel takes over, a buffer sized at 80 rows (ternary 11264 x 11008: 0 bytes) failed at 33 (6.4 MB),
+// kernel takes over, a buffer sized at 80 rows (ternary 11264 x 11008: 0 bytes) failed at 20 (4.3 MB),
 // one sized at 1024 rows (3328 x 512) at every smaller M.
 enum class Kind { kDecode, kLockstep, kPrefill, kResident, kRows };
 struct Plan {
@@ -312,8 +312,8 @@ struct Plan {
 };
 
 // cap: the largest workspace the plan may use (the no-allocation entry point's scratch).
-// dtype: the activation type (the prefill tile width depends on it, the workspace does not,
-// so the workspace queries plan without it).
+// dtype: the activation type (the prefill tiles and the line between row tiles and lockstep kernel
+// depend on it, `need` does not, so the workspace queries plan without it).
 Plan make_plan(int fmt, const hq::GemmDesc& d, size_t cap = SIZE_MAX, int dtype = HQ_DTYPE_F16) {
   Plan p{};
   if (d.M > decode_max_m()) {
@@ -330,7 +330,7 @@ Plan make_plan(int fmt, const hq::GemmDesc& d, size_t cap = SIZE_MAX, int dtype 
     if (d.gen) p.need = std::max(p.use, lockstep_need());
     return p;
   }
-  p.rc = hq::choose_rows(fmt, d, cap);
+  p.rc = hq::choose_rows(fmt, d, cap, dtype);
   if (p.rc.ok) {
     p.kind = Kind::kRows;
     p.use = hq::rows_workspace_bytes(d, p.rc);
@@ -346,7 +346,9 @@ Plan make_plan(int fmt, const hq::GemmDesc& d, size_t cap = SIZE_MAX, int dtype 
   // The lockstep kernel takes every decode shape; under a cap with fewer pieces per slab.
   p.kind = Kind::kLockstep;
   p.lc = hq::choose_decode_ls(fmt, d, cap);
+  p.lc.fold = !p.rc.long_k;
   p.use = p.need = hq::decode_ls_workspace_bytes(d, p.lc);
+  if (p.rc.long_k) p.need = std::max(p.use, std::min(cap, hq::rows_workspace_bytes(d, p.rc)));  // the other type's plan
   return p;
 }
 
@@ -551,9 +553,10 @@ std::string describe(int fmt, int dtype, const hq::GemmDesc& d, const Plan& p) {
   } else if (p.kind == Kind::kLockstep) {
     std::snprintf(b, sizeof b,
                   "hq_decode_ls_kernel<%s,%s,KG=%d,GW=%d,T=%d,U=%d,MT=%d%s> grid=%d pieces x slabs of %d tiles, "
-                  "%d wavefronts%s ws=%zu",
+                  "%d wavefronts%s%s ws=%zu",
                   fmt_name(fmt), dt_name(dtype), p.lc.KG, p.lc.GW, p.lc.T, p.lc.U, p.lc.MT, d.gen ? ",general" : "",
-                  p.lc.S, p.lc.SW, p.lc.KG * p.lc.GW, p.lc.P > 0 ? " balanced grid" : "", p.need);
+                  p.lc.S, p.lc.SW, p.lc.KG * p.lc.GW, p.lc.P > 0 ? " balanced grid" : "",
+                  !p.lc.fold && fmt == HQ_FORMAT_INT4 && dtype == HQ_DTYPE_F16 && p.lc.MT == 5 ? " fp32 scales" : "", p.need);
   } else {
     int n = std::snprintf(b, sizeof b, "hq_prefill_kernel<%s,%s%s>", fmt_name(fmt), dt_name(dtype),
                           d.gen ? ",general" : "");

@@ -148,7 +148,7 @@ __device__ __forceinline__ void ls_tie(u4& a) { asm volatile("" : "+v"(a)); }
 __device__ __forceinline__ void ls_tie(u2& a) { asm volatile("" : "+v"(a)); }
 __device__ __forceinline__ void ls_tie(uint32_t& a) { asm volatile("" : "+v"(a)); }
 
-template <int FMT, int DT, int KG, int GW, int T, int U, int MT, bool FUSED, bool GEN, bool BAL = false>
+template <int FMT, int DT, int KG, int GW, int T, int U, int MT, bool FUSED, bool GEN, bool BAL = false, bool FOLD = true>
 __global__ void __launch_bounds__(64 * KG * GW, KG == 1 && MT > 1 ? 2 : 1)
     hq_decode_ls_kernel(const GemmDesc d, const LsPlan pl) {
   static_assert(!BAL || (KG > 1 && !GEN), "the balanced grid is for the fast kernels with two k-groups");
@@ -172,8 +172,11 @@ __global__ void __launch_bounds__(64 * KG * GW, KG == 1 && MT > 1 ? 2 : 1)
   // the per-k-block sums (40 VGPRs) that would not fit beside the fragments are not needed.
   // Measured on MI355X (5120 x 27648, M = 80): 36.2 -> 35.0 us. With fewer row tiles, or
   // ternary weights, scaling each k-block's sums in fp32 measured as fast or faster (one
-  // v_pk_mul_f16 per fragment word against MT x T x 4 FMAs per k-block).
-  constexpr bool kFold = !GEN && DT == HQ_DTYPE_F16 && kInt4 && MT == 5;
+  // v_pk_mul_f16 per fragment word against MT x T x 4 FMAs per k-block). FOLD = false keeps the fp32
+  // scaling (its sums fit: 228 VGPRs) for the calls whose pieces are too long for the shared row tiles,
+  // which scale in fp32: error against 64 bits 2.1e-4 where the folded weights have 2.8e-4, at 3-8% more time
+  // (130 slabs of four tiles over K = 19456, M = 80: folded 46.2 us, fp32 48.7, row tiles 63.8).
+  constexpr bool kFold = FOLD && !GEN && DT == HQ_DTYPE_F16 && kInt4 && MT == 5;
   // Several row tiles: every A fragment of a k-block is read before the first wait, and the
   // weight fragments are dequantised while those reads are in flight (a wait per row tile
   // left the LDS latency exposed MT times per step). Measured on MI355X: ternary 5120 x 34816
@@ -851,7 +854,7 @@ uint32_t ls_assign_slabs(GemmDesc& d, uint32_t sw) {
   return g;
 }
 
-template <int FMT, int DT, int KG, int GW, int T, int U, int MT, bool GEN = false>
+template <int FMT, int DT, int KG, int GW, int T, int U, int MT, bool GEN = false, bool FOLD = true>
 hipError_t ls_launch_t(GemmDesc d, const LsConfig& c, void* ws, uint32_t* fault, uint32_t spin, hipStream_t stream) {
   const bool fused = d.nseg > 1;
   if (d.M > 16u * MT) return hipErrorInvalidValue;
@@ -871,7 +874,7 @@ hipError_t ls_launch_t(GemmDesc d, const LsConfig& c, void* ws, uint32_t* fault,
     pl.part = reinterpret_cast<float*>(static_cast<char*>(ws) + kCounterBytes);
   }
   if (c.P > 0) {  // balanced grid
-    if constexpr (GEN || KG == 1 || (MT == 1 && !(KG == 2 && GW == 4 && T == 2 && U == 2))) {
+    if constexpr (GEN || !FOLD || KG == 1 || (MT == 1 && !(KG == 2 && GW == 4 && T == 2 && U == 2))) {
       return hipErrorInvalidConfiguration;
     } else {
       const uint32_t P = (uint32_t)c.P;
@@ -904,10 +907,10 @@ hipError_t ls_launch_t(GemmDesc d, const LsConfig& c, void* ws, uint32_t* fault,
     hipLaunchKernelGGL((hq_decode_ls_kernel<FMT, DT, KG, GW, T, U, MT, true, true>), dim3(pl.S, G), dim3(64 * KG * GW),
                        0, stream, d, pl);
   } else if (fused) {
-    hipLaunchKernelGGL((hq_decode_ls_kernel<FMT, DT, KG, GW, T, U, MT, true, false>), dim3(pl.S, G),
+    hipLaunchKernelGGL((hq_decode_ls_kernel<FMT, DT, KG, GW, T, U, MT, true, false, false, FOLD>), dim3(pl.S, G),
                        dim3(64 * KG * GW), 0, stream, d, pl);
   } else {
-    hipLaunchKernelGGL((hq_decode_ls_kernel<FMT, DT, KG, GW, T, U, MT, false, false>), dim3(pl.S, G),
+    hipLaunchKernelGGL((hq_decode_ls_kernel<FMT, DT, KG, GW, T, U, MT, false, false, false, FOLD>), dim3(pl.S, G),
                        dim3(64 * KG * GW), 0, stream, d, pl);
   }
   return hipGetLastError();
@@ -943,7 +946,10 @@ hipError_t ls_launch_fd(const GemmDesc& d, const LsConfig& c, void* ws, uint32_t
       case 2: return ls_launch_t<FMT, DT, 2, 4, 2, 2, 2>(d, c, ws, fault, spin, stream);
       case 3: return ls_launch_t<FMT, DT, 2, 4, 2, 2, 3>(d, c, ws, fault, spin, stream);
       case 4: return ls_launch_t<FMT, DT, 2, 4, 2, 2, 4>(d, c, ws, fault, spin, stream);
-      case 5: return ls_launch_t<FMT, DT, 2, 4, 2, 2, 5>(d, c, ws, fault, spin, stream);
+      case 5:
+        if constexpr (FMT == HQ_FORMAT_INT4 && DT == HQ_DTYPE_F16)
+          if (!c.fold) return ls_launch_t<FMT, DT, 2, 4, 2, 2, 5, false, false>(d, c, ws, fault, spin, stream);
+        return ls_launch_t<FMT, DT, 2, 4, 2, 2, 5>(d, c, ws, fault, spin, stream);
       default: return hipErrorInvalidConfiguration;
     }
   }

@@ -111,6 +111,7 @@ struct LsConfig {
   int MT;  // 16-row tiles of activations (1 .. kLsMaxRowTiles): rows M <= 16 MT
   int P = 0;  // balanced grid (several row tiles, more slabs than CUs): P workgroups, each an
               // equal run of (slab, k-block) units; 0 = the S-piece grid
+  bool fold = true;  // int4, fp16, five row tiles: the group scale goes into the fp16 weights (false: fp32 sums)
 };
 // The lockstep kernel takes up to this many 16-row tiles (M <= 80: a split-fuse step of 16
 // decode tokens and a 64-token prefill chunk fits one call).
@@ -144,9 +145,10 @@ hipError_t launch_decode_ls(int fmt, int dtype, GemmDesc d, const LsConfig& c, v
 // Shared row tiles (hq_rows.hip, 17 <= M <= 80): slabs of four column tiles, S pieces along K.
 struct RowsConfig {
   int S;
-  bool ok;  // the kernel takes the call
+  bool ok;            // the kernel takes the call
+  bool long_k = false;  // only the length of its pieces keeps the kernel off
 };
-RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MAX);
+RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap = SIZE_MAX, int dtype = HQ_DTYPE_F16);
 size_t rows_workspace_bytes(const GemmDesc& d, const RowsConfig& c);
 hipError_t launch_rows(int fmt, int dtype, const GemmDesc& d, const RowsConfig& c, void* ws, hipStream_t stream);
 

@@ -386,32 +386,39 @@ hipError_t rows_mt(const GemmDesc& d, const RowsConfig& c, void* ws, hipStream_t
 }  // namespace
 
 // The longest piece, in k-blocks, at which slabs of four tiles in S pieces still beat the lockstep
-// kernel: what they save is spent once a launch, and over a long piece its slabs of eight tiles, cut
-// finer, keep more of the chip busy. MI355X, lockstep -> this kernel at k-blocks, weights from memory,
-// ternary fp16 unless noted:
-//  * lockstep grids past one workgroup per CU (171-184 slabs here): 172 slabs M = 56 88 35.8 -> 32.3 us,
-//    int4 bf16 M = 80 176 110.5 -> 76.4, but ternary M = 33 88 27.9 -> 29.0;
-//  * lockstep workgroups with at most 6/7 of the work of ours (81-102 and 129-170 slabs, which leave
-//    CUs idle here): 130 slabs M = 56 32 15.7 -> 14.0, 48 18.6 -> 19.4, 96 27.2 -> 33.6, 152 37.9 -> 51.9;
-//    M = 80 48 22.5 -> 21.2, 96 33.1 -> 37.0;
-//  * as much work: 256 slabs M = 33 96 29.1 -> 30.9, M = 56 35.5 -> 34.6, M = 80 44.8 -> 38.7; past the
-//    limits 2-10% slower; lower in pieces, which meet through memory.
-uint32_t rows_max_piece(int fmt, const GemmDesc& d, uint32_t S, size_t ws_cap) {
-  const uint32_t mt = (d.M + 15u) / 16u, cus = (uint32_t)cu_count();
+// kernel, by the type and the row tiles (2 .. 5): what they save is spent once a launch, and over a long
+// piece its slabs of eight tiles, cut finer, keep more of the chip busy. Four kinds of grids: lockstep's
+// past one workgroup per CU (171-184 slabs here); its workgroups with under 6/7 of the work of ours (81-102 and
+// 129-170 slabs, which leave CUs idle here); as much work, whole slabs; in pieces. Fitted to 22,000 pairs on
+// MI355X (80 slab counts of 16..256, 8..216 k-blocks, weights from memory), each within 5% of the faster
+// kernel, nearly all within 2%; int4 fp16 at 65 to 80 rows is held against lockstep with fp32 scales (with them
+// in the fp16 weights it is up to 9% faster than this kernel past 140 k-blocks). Lockstep -> this kernel, us: 172 slabs, 176 k-blocks int4 bf16 M = 80 110.5 -> 76.4; 130
+// slabs ternary fp16 M = 56 32 15.7 -> 14.0, 48 18.6 -> 19.4, 152 37.9 -> 51.9, M = 80 48 22.5 -> 21.2, 96 33.1 ->
+// 37.0; 256 slabs, 96 ternary M = 33 29.1 -> 30.9, M = 80 44.8 -> 38.7, int4 bf16 152 M = 80 86.5 -> 76.5.
+constexpr uint16_t kAny = 0xFFFF;
+constexpr uint16_t kMaxPiece[4][3][4] = {
+    // int4 fp16, int4 bf16, ternary
+    {{kAny, kAny, kAny, kAny}, {kAny, kAny, kAny, kAny}, {36, 96, kAny, kAny}},
+    {{20, 32, 46, 52}, {20, 40, 46, 64}, {20, 32, 46, 64}},
+    {{36, 64, 96, 216}, {36, 96, 152, kAny}, {36, 64, 96, 176}},
+    {{24, 48, 80, kAny}, {24, kAny, kAny, kAny}, {24, 46, 80, kAny}},
+};
+bool rows_piece_too_long(int fmt, int dtype, const GemmDesc& d, uint32_t S, size_t ws_cap) {
   uint32_t slabs = 0;
   for (uint32_t i = 0; i < d.nseg; ++i) slabs += (d.seg[i].ntiles + 7u) / 8u;
   const uint32_t pieces = (uint32_t)choose_decode_ls(fmt, d, ws_cap, false).S;
-  if (slabs * pieces > cus) return fmt == HQ_FORMAT_INT4 || mt >= 4u ? ~0u : mt == 2u ? 32u : 64u;
-  if (7u * S <= 3u * pieces) return mt == 2u ? 20u : mt == 3u ? 24u : mt == 4u ? 40u : 48u;
-  if (S == 1u) return mt == 2u ? 40u : mt == 3u ? 64u : mt == 4u ? 96u : 128u;
-  return mt == 2u ? 24u : mt == 3u ? 40u : mt == 4u ? 80u : 96u;
+  const int grid = slabs * pieces > (uint32_t)cu_count() ? 0 : 7u * S < 3u * pieces ? 1 : S == 1u ? 2 : 3;
+  const int type = fmt != HQ_FORMAT_INT4 ? 2 : dtype == HQ_DTYPE_F16 ? 0 : 1;
+  uint32_t most = kMaxPiece[grid][type][(d.M + 15u) / 16u - 2u];
+  if (grid == 3 && 2u * S < pieces && d.M <= 64u) most = std::min(most, 64u);  // 69-72 slabs, 72 k-blocks ternary M = 56 33.3 -> 36.0 us
+  return most != kAny && (d.nkb + S - 1u) / S > most;
 }
 
 // Taken when the slabs number at most the CUs, cut into as many pieces (at most eight, each at
 // least one step per k-group) as stay within one workgroup per CU and fill half of them. Measured on
 // MI355X at G x S workgroups, M = 20..80, ternary and int4, fp16 and bf16: 2-113% faster than the
 // lockstep kernel (most at few slabs: 1024 x 4096 M = 80 18.1 -> 8.6 us), except, kept there: pieces too
-// long for their grid (rows_max_piece), grids
+// long for their grid (kMaxPiece), grids
 // under two thirds of the CUs at few rows (5120 x 9000, 141 slabs: M = 20 11.8 against 13.2, M = 33 14.4
 // against 15.0; M = 64 18.0 -> 17.0), a long K at few rows (17408 x 5120: M = 20 16.0 against 17.1, M = 33
 // 19.9 -> 19.4), and int4 up to 32 rows, where lockstep's balanced grids run the wide shapes (5120 x
@@ -419,7 +426,7 @@ uint32_t rows_max_piece(int fmt, const GemmDesc& d, uint32_t S, size_t ws_cap) {
 // = 80 50.7 against 53.4).
 // HQ_ROWS = 0 keeps the lockstep kernel, a number forces that many pieces (tuning and tests); any
 // lockstep override keeps it too.
-RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap) {
+RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap, int dtype) {
   RowsConfig c{1, false};
   if (d.M <= 16u || d.M > 80u || d.gen) return c;
   const char* e = std::getenv("HQ_ROWS");
@@ -440,7 +447,8 @@ RowsConfig choose_rows(int fmt, const GemmDesc& d, size_t ws_cap) {
     const uint32_t wgs = G * (uint32_t)c.S;
     if (2u * wgs < cus || (3u * wgs < 2u * cus && d.M <= 48u && G > cus / 2u)) return c;
     if (d.nkb > (d.M <= 32u ? 64u : d.M <= 48u ? 144u : ~0u)) return c;
-    if ((d.nkb + (uint32_t)c.S - 1u) / (uint32_t)c.S > rows_max_piece(fmt, d, (uint32_t)c.S, ws_cap)) return c;
+    c.long_k = rows_piece_too_long(fmt, dtype, d, (uint32_t)c.S, ws_cap);
+    if (c.long_k) return c;
   }
   c.ok = rows_workspace_bytes(d, c) <= ws_cap;
   return c;

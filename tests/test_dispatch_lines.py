@@ -18,15 +18,24 @@ def plan(fmt, dt, M, K, N, **kw):
 # Shared row tiles: slabs of four tiles that leave CUs idle lose over a long K, by rows.
 @pytest.mark.parametrize("fmt,M,slabs,kblocks,rows", [
     (T2, 56, 130, 32, True), (T2, 56, 130, 48, False), (T2, 80, 130, 48, True), (T2, 80, 130, 96, False),
-    (I4, 64, 160, 152, False), (I4, 56, 136, 151, False), (I4, 80, 86, 128, False), (T2, 33, 86, 48, True),
+    (I4, 64, 160, 152, False), (I4, 56, 136, 151, False), (I4, 80, 86, 96, True), (I4, 80, 86, 128, False), (T2, 33, 86, 48, True),
     (T2, 33, 86, 96, False), (T2, 20, 86, 32, True), (T2, 20, 86, 64, False),
-    (I4, 80, 172, 176, True), (T2, 56, 184, 128, True), (T2, 33, 172, 88, False),  # past one lockstep workgroup per CU
+    (I4, 80, 172, 176, True), (T2, 56, 184, 128, True), (T2, 33, 172, 88, True), (T2, 33, 172, 112, False),  # past one lockstep workgroup per CU
     (T2, 20, 256, 32, True), (T2, 20, 256, 48, False), (T2, 33, 256, 64, True), (T2, 33, 256, 96, False),
-    (T2, 56, 256, 96, True), (I4, 80, 256, 112, True), (I4, 80, 240, 176, False),
+    (T2, 56, 256, 96, True), (I4, 80, 256, 112, True), (I4, 80, 240, 176, True), (T2, 80, 240, 192, False), (T2, 33, 86, 64, True),
     (I4, 80, 32, 216, True), (T2, 56, 16, 216, True),                              # few slabs in eight pieces
 ])
 def test_row_tiles_by_piece_length(fmt, M, slabs, kblocks, rows):
     assert plan(fmt, F16, M, 128 * kblocks, 64 * slabs).startswith("hq_rows_kernel<" if rows else "hq_decode_ls_kernel<")
+
+
+def test_row_tiles_by_type():
+    # Int4 with bf16, whose lockstep kernel carries a correction chain, keeps the row tiles longer; what a call
+    # asks for is the same for both types.
+    for M, kblocks, slabs in ((40, 88, 240), (56, 112, 240), (40, 88, 86)):
+        f, b = (plan(I4, dt, M, 128 * kblocks, 64 * slabs) for dt in (F16, BF16))
+        assert f.startswith("hq_decode_ls_kernel<") and b.startswith("hq_rows_kernel<"), (f, b)
+        assert f.split(" ws=")[1] == b.split(" ws=")[1]
 
 
 # Whole 64 x 128 prefill tiles against the K split over workgroups: from how many tiles, by K and type.
@@ -67,3 +76,10 @@ def test_general_resident_slabs(M, kblocks, N, resident):
     assert d.startswith("hq_decode_xr_kernel<" if resident else "hq_decode_ls_kernel<"), d
     if (M, kblocks, N) == (16, 8, 24576):  # two workgroups of four wavefronts per CU
         assert "x 4 wavefronts" in d
+
+
+def test_lockstep_keeps_fp32_scales_where_the_row_tiles_would_have_them():
+    # Int4, fp16, 65 to 80 rows: a piece too long for the row tiles must not round its weights times their scales.
+    assert " fp32 scales" in plan(I4, F16, 80, 19456, 8320)
+    for fmt, dt, M, K, N in ((I4, F16, 80, 5120, 34816), (I4, BF16, 80, 19456, 8320), (I4, F16, 64, 19456, 8320)):
+        assert plan(fmt, dt, M, K, N).startswith("hq_decode_ls_kernel<") and " fp32 scales" not in plan(fmt, dt, M, K, N)

@@ -66,13 +66,13 @@ def test_graph_replays_equal_eager(cuda, label, fmt, xdt, M, K, N, plan):
 
 
 def test_capture_after_a_warm_up_of_more_rows(cuda):
-    # Ternary 11264 x 11008 runs whole slabs at 80 rows and K pieces at 33: the call of 80 rows leaves the
+    # Ternary 11264 x 11008 runs whole slabs at 80 rows and K pieces at 20: the call of 80 rows leaves the
     # stream's library workspace large enough for the other, which is then captured as it comes.
     import torch
 
     K, N = 11264, 11008
     assert "hq_rows_kernel<ternary2,f16,MT=5> grid=1 pieces" in hq.describe(O.TERNARY2, O.F16, 80, K, N)
-    P = O.Problem(O.TERNARY2, 33, K, N, 128, O.F16, seed=9990)
+    P = O.Problem(O.TERNARY2, 20, K, N, 128, O.F16, seed=9990)
     D = DeviceProblem(P)
     y0 = D.run()
     side, out = torch.cuda.Stream(), torch.empty_like(y0)

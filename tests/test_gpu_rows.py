@@ -1,9 +1,10 @@
 """GPU tests of the shared-row-tile kernel (17 <= M <= 80): every row-tile count, format and type, pieces
 along K, k-groups without k-blocks, ragged columns, segments, strides, and the plans the library picks."""
+import numpy as np
 import pytest
 
 import oracle as O
-from gpu_util import DeviceProblem, to_dev_u16
+from gpu_util import DeviceProblem, to_dev_u16, to_host_f32
 from nebula_amd import hq
 from test_gpu_parity import check, torch_equal
 
@@ -46,10 +47,36 @@ def test_default_plans(cuda, fmt, M, K, N, group, rows):
         check(DeviceProblem(P).run(), P.reference(threads=16), O.BF16, f"rows default M={M} K={K} N={N}", P)
 
 
+# Pieces one k-block too long for the row tiles: the lockstep kernel, whose int4 fp16 form at five row tiles keeps
+# the scales in fp32 there. Its error in the 2-norm is the rounding of the outputs to fp16, uniform over an ulp: 2^-10 /
+# sqrt(12) of the binade's foot, 1.9e-4 to 2.1e-4 of the values. Rounding the products of weight and scale adds as
+# much again, independently, 2.8e-4 in all: the line is halfway.
+@pytest.mark.parametrize("M,Ns", [(65, [8250]), (80, [8250]), (80, [5000, 1000, 2250])])
+def test_long_pieces_keep_fp32_scales(cuda, M, Ns):
+    import torch
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the boundaries are those of a 256-CU device")
+    K = 128 * 65
+    if len(Ns) == 1:
+        assert " fp32 scales" in hq.describe(O.INT4, O.F16, M, K, Ns[0])
+    probs = [O.Problem(O.INT4, M, K, n, 128, O.F16, seed=9640 + i) for i, n in enumerate(Ns)]
+    for p in probs:
+        p.X = probs[0].X
+    devs = [DeviceProblem(p) for p in probs]
+    segs = [(d.Wp, d.S, d.P.N) for d in devs]
+    outs = hq.gemm_fused(O.INT4, devs[0].X, segs)
+    for p, y, z in zip(probs, outs, hq.gemm_fused(O.INT4, devs[0].X, segs)):
+        assert torch_equal(y, z)  # one order of sums
+        ref = p.reference(threads=16)
+        check(y, ref, O.F16, f"fp32 scales M={M} N={p.N}", p)
+        e = to_host_f32(y).astype(np.float64) - ref
+        assert np.linalg.norm(e) <= 2.4e-4 * np.linalg.norm(ref.astype(np.float64))
+
+
 def test_non_finite_scales_strides_and_counters(cuda, monkeypatch):
     # Ternary groups without a finite scale drop out; X and Y have row strides of their own; a caller
     # workspace is left with zero counters and serves two calls.
-    import numpy as np
     import torch
 
     monkeypatch.setenv("HQ_ROWS", "3")

@@ -45,14 +45,14 @@ def test_prefill_asks_for_what_the_256_column_plan_does(monkeypatch, fmt, K, Ns,
 
 
 def test_a_plan_that_writes_nothing_takes_any_workspace():
-    # Ternary 11264 x 11008 at 80 rows runs whole slabs: it asks for what 33 rows need, but does not refuse
-    # a smaller buffer. At 33 rows, pieces: one byte less is refused (before any launch).
+    # Ternary 11264 x 11008 at 80 rows runs whole slabs: it asks for what 20 rows need, but does not refuse
+    # a smaller buffer. At 20 rows, pieces: one byte less is refused (before any launch).
     L = hq.lib()
     K, N = 11264, 11008
-    big, small = need(hq.FORMAT_TERNARY2, 80, K, [N]), need(hq.FORMAT_TERNARY2, 33, K, [N])
+    big, small = need(hq.FORMAT_TERNARY2, 80, K, [N]), need(hq.FORMAT_TERNARY2, 20, K, [N])
     assert big >= small > 0
     assert "hq_rows_kernel" in hq.describe(hq.FORMAT_TERNARY2, hq.DTYPE_F16, 80, K, N)
     segs = (hq.Segment * 1)(hq.Segment(0x2000, 0x3000, None, 0x4000, N, N))
-    args = (0x1000, hq.DTYPE_F16, K, hq.FORMAT_TERNARY2, segs, 1, 33, K, 128)
+    args = (0x1000, hq.DTYPE_F16, K, hq.FORMAT_TERNARY2, segs, 1, 20, K, 128)
     assert L.hq_gemm_fused(*args, ctypes.c_void_p(0x10000), small - 1, None) == hq.HQ_ERR_WORKSPACE
     assert L.hq_gemm_fused(*args, ctypes.c_void_p(0x10010), big, None) == hq.HQ_ERR_ALIGNMENT
