@@ -392,9 +392,10 @@ hipError_t rows_mt(const GemmDesc& d, const RowsConfig& c, void* ws, hipStream_t
 // 129-170 slabs, which leave CUs idle here); as much work, whole slabs; in pieces. Fitted to 22,000 pairs on
 // MI355X (80 slab counts of 16..256, 8..216 k-blocks, weights from memory), each within 5% of the faster
 // kernel, nearly all within 2%; int4 fp16 at 65 to 80 rows is held against lockstep with fp32 scales (with them
-// in the fp16 weights it is up to 9% faster than this kernel past 140 k-blocks). Lockstep -> this kernel, us: 172 slabs, 176 k-blocks int4 bf16 M = 80 110.5 -> 76.4; 130
-// slabs ternary fp16 M = 56 32 15.7 -> 14.0, 48 18.6 -> 19.4, 152 37.9 -> 51.9, M = 80 48 22.5 -> 21.2, 96 33.1 ->
-// 37.0; 256 slabs, 96 ternary M = 33 29.1 -> 30.9, M = 80 44.8 -> 38.7, int4 bf16 152 M = 80 86.5 -> 76.5.
+// in the fp16 weights it is up to 9% faster than this kernel past 140 k-blocks). Lockstep -> this kernel, us,
+// by k-blocks: 172 slabs int4 bf16 M = 80 176 110.5 -> 76.4; 130 slabs ternary fp16 M = 56 32 15.7 -> 14.0, 48
+// 18.6 -> 19.4, 152 37.9 -> 51.9, M = 80 48 22.5 -> 21.2, 96 33.1 -> 37.0; 256 slabs ternary M = 33 96 29.1 ->
+// 30.9, M = 80 44.8 -> 38.7, int4 bf16 M = 80 152 86.5 -> 76.5.
 constexpr uint16_t kAny = 0xFFFF;
 constexpr uint16_t kMaxPiece[4][3][4] = {
     // int4 fp16, int4 bf16, ternary
@@ -410,7 +411,8 @@ bool rows_piece_too_long(int fmt, int dtype, const GemmDesc& d, uint32_t S, size
   const int grid = slabs * pieces > (uint32_t)cu_count() ? 0 : 7u * S < 3u * pieces ? 1 : S == 1u ? 2 : 3;
   const int type = fmt != HQ_FORMAT_INT4 ? 2 : dtype == HQ_DTYPE_F16 ? 0 : 1;
   uint32_t most = kMaxPiece[grid][type][(d.M + 15u) / 16u - 2u];
-  if (grid == 3 && 2u * S < pieces && d.M <= 64u) most = std::min(most, 64u);  // 69-72 slabs, 72 k-blocks ternary M = 56 33.3 -> 36.0 us
+  // Pieces just short of lockstep's (69-72 slabs in three): 72 k-blocks each ternary M = 56 27.9 -> 30.2 us.
+  if (grid == 3 && 2u * S < pieces && d.M <= 64u) most = std::min(most, 64u);
   return most != kAny && (d.nkb + S - 1u) / S > most;
 }
 

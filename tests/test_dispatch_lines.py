@@ -32,7 +32,7 @@ def test_row_tiles_by_piece_length(fmt, M, slabs, kblocks, rows):
 def test_row_tiles_by_type():
     # Int4 with bf16, whose lockstep kernel carries a correction chain, keeps the row tiles longer; what a call
     # asks for is the same for both types.
-    for M, kblocks, slabs in ((40, 88, 240), (56, 112, 240), (40, 88, 86)):
+    for M, kblocks, slabs in ((40, 88, 240), (56, 112, 240), (40, 76, 86)):
         f, b = (plan(I4, dt, M, 128 * kblocks, 64 * slabs) for dt in (F16, BF16))
         assert f.startswith("hq_decode_ls_kernel<") and b.startswith("hq_rows_kernel<"), (f, b)
         assert f.split(" ws=")[1] == b.split(" ws=")[1]
