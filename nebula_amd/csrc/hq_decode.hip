@@ -1243,8 +1243,8 @@ XrConfig choose_decode_xr(int fmt, const GemmDesc& d, size_t ws_cap) {
       // int4 4096 x 40960 22.8 -> 17.4 us; at 1.7 rounds (5120 x 55296) 8-tile slabs stay
       // ahead from M = 4. The general kernels stop short of that: there the lockstep kernel's slabs
       // of eight tiles cover three quarters of the CUs and run whole (1024 x 24576 M = 16 9.2 against
-      // 12.2 us, 3072 x 24576 18.6 against 20.4; at 368 slabs here 12-22% faster).
-      const bool t4_spill = t == 4 && (d.gen ? 2u * wgs < 3u * cus * per_cu : 2u * wgs <= 3u * cus * per_cu);
+      // 12.2 us, 3072 x 24576 18.6 against 20.4; at 368 slabs here 12-22% faster, over K = 8192 6-10%).
+      const bool t4_spill = t == 4 && (d.gen && d.nkb < 48u ? 2u * wgs < 3u * cus * per_cu : 2u * wgs <= 3u * cus * per_cu);
       if (per_cu < 1 || (wgs > cus * per_cu && !t4_spill)) continue;
       // Whole slabs leaving more than half of the CUs idle: try a split first.
       if (s == 1 && wgs * 2u < cus && total_slabs(d, t) * 2u <= cus * per_cu && d.nkb >= 2 && d.M <= 4u) break;

@@ -975,6 +975,42 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
   return l;
 }
 
+// Microseconds of a prefill call of at most one 64 x 128 tile per CU as 256-column tiles of 64 rows in `ways`
+// equal ranges of K (stream-K), and as whole 64 x 128 tiles of four K groups, MI355X. Whole tiles take time by
+// K and, through the memory behind them, by their number. The split takes it by a range's length
+// times the workgroups that share a CU, by the grid, and by the ways: a tile's last workgroup adds up one partial
+// tile for each, ranges that do not divide K add more (a workgroup's first and last tile are then shared), and
+// rows that are not 16-byte aligned are stored element by element. Fitted to 2,321 shapes for each row (17..216
+// k-blocks, 81..1092 rows, 16..256 tiles, half of them of models' widths), to 3% for whole tiles and 8% for the
+// split: the plan it picks needs 0.2-0.3% more than the faster one on average. A line by tiles and K alone took
+// 1-12% more, up to twice the time, since the split's time follows how K divides.
+struct SmallTileCost {
+  float s0, s_len, s_grid, s_way, s_way_grid, s_rest_way, s_rest_grid, s_ragged;  // split
+  float w0, w_len, w_mem;                                                         // whole
+};
+constexpr SmallTileCost kSmallTileCost[2][2][2] = {
+    // [int4, ternary][fp16, bf16][fast, general]
+    {{{10.90f, 1.141f, 2.90f, 0.515f, 0.128f, 0.334f, 0.29f, 0.446f, 8.60f, 0.365f, 0.149f},
+      {11.61f, 1.357f, 2.19f, 0.577f, 0.106f, 0.348f, 0.27f, 0.467f, 9.11f, 0.433f, 0.119f}},
+     {{11.47f, 1.444f, 2.18f, 0.580f, 0.096f, 0.350f, -0.14f, 0.481f, 8.46f, 0.562f, 0.123f},
+      {12.42f, 1.635f, 1.87f, 0.598f, 0.092f, 0.335f, 0.02f, 0.460f, 9.01f, 0.621f, 0.101f}}},
+    {{{14.57f, 0.897f, -0.18f, 0.305f, 0.355f, 0.218f, 2.13f, 0.545f, 8.42f, 0.363f, 0.100f},
+      {15.36f, 0.939f, -0.66f, 0.290f, 0.375f, 0.224f, 2.16f, 0.582f, 8.75f, 0.410f, 0.075f}},
+     {{14.48f, 0.906f, -0.14f, 0.288f, 0.363f, 0.225f, 1.99f, 0.571f, 8.69f, 0.381f, 0.087f},
+      {15.21f, 0.939f, -0.52f, 0.296f, 0.370f, 0.229f, 2.13f, 0.583f, 8.75f, 0.425f, 0.061f}}},
+};
+float whole_over_split(int fmt, int dtype, const GemmDesc& d, const PrefillLaunch& cur, uint32_t t64, uint32_t cus) {
+  const SmallTileCost& c = kSmallTileCost[fmt == HQ_FORMAT_INT4 ? 0 : 1][dtype == HQ_DTYPE_F16 ? 0 : 1][d.gen ? 1 : 0];
+  const uint32_t ways = std::max(1u, cur.psk / cur.tiles), len = (d.nkb + ways - 1u) / ways;
+  bool ragged = false;
+  for (uint32_t i = 0; i < d.nseg; ++i) ragged |= d.seg[i].N % 8u != 0u;
+  const float grid = (float)cur.psk / (float)cus, n = (float)ways, rest = d.nkb % ways ? 1.f : 0.f;
+  const float split = c.s0 + c.s_len * (float)(len * ((cur.psk + cus - 1u) / cus)) + c.s_grid * grid +
+                      n * (c.s_way + c.s_way_grid * grid) + rest * (c.s_rest_way * n + c.s_rest_grid * grid) +
+                      (ragged ? c.s_ragged * n : 0.f);
+  return (c.w0 + (float)d.nkb * (c.w_len + c.w_mem * (float)t64 / (float)cus)) / split;
+}
+
 // 128-column whole tiles for grids that are small beside the chip, in place of the plan over
 // 256-column tiles (`cur`), and the general kernels' 128-row tiles for large ones. Such grids
 // left CUs idle or split their tiles along K over workgroups, paying for partial tiles in
@@ -985,17 +1021,10 @@ PrefillLaunch make_whole(int RT, int KS, int TW, const GemmDesc& d) {
 // Measured on MI355X (K = 4096, previous plan -> this one, int4 fp16 / int4 bf16 / ternary fp16):
 //  * 64 x 128 tiles at most one per CU, four groups: M = 128, N = 14336 (224 tiles) 49.8 -> 23.4 /
 //    52.2 -> 27.3 / 30.5 -> 21.1 us; M = 333, N = 4096 (192) 46.0 -> 20.3 / 46.6 -> 26.4 / 35.4 ->
-//    19.0; M = 81, N = 4096 (64) 24.1 -> 19.4 / 26 -> 25.6 / 24.6 -> 18.5. Their time grows with K
-//    alone, that of a K split over workgroups with the work, so the line rises with K: at 64
-//    k-blocks (K = 8192) 64 tiles 37.4 -> 33.0 but 32 tiles 26.3 -> 32.3; at 216 (K = 27648)
-//    int4 240 tiles 126 -> 114, 120 tiles 92 -> 97, ternary 240 109 -> 104, 120 68 -> 94; at 112
-//    (K = 14336) 128 tiles int4 70 -> 57, ternary 46 -> 52. Int4 with bf16, whose weights take more
-//    VALU in the half as high tiles, from more tiles on: at 28 k-blocks 72 tiles 21.9 -> 24.2, 80 14% faster; at
-//    64 80 tiles 42.3 -> 45.2, 88 7% faster; at 112 112 tiles 62.1 -> 74.4, 152 7% faster; at 216 160 tiles
-//    116 -> 138, 248 12% faster. Ternary past 64 k-blocks: at 80 96 tiles fp16 34.6 -> 39.0, bf16 38.5 -> 40.2, 104 6
-//    and 13% faster; at 88 fp16 124 tiles 40.1 -> 44.1, 136 2-17% faster; in groups of 64 from a few more (at 150
-//    186 tiles 72.0 -> 76.4). Below
-//    17 k-blocks two groups do (K = 1024, M = 384, N = 4096: 16.5 -> 8.9 us, four groups 9.7).
+//    19.0; M = 81, N = 4096 (64) 24.1 -> 19.4 / 26 -> 25.6 / 24.6 -> 18.5; against the K split by cost
+//    (kSmallTileCost), since that depends on how K divides: int4 bf16 62.1 -> 74.4 us at K = 14336, N = 7168, M
+//    = 81 (16 ways of seven k-blocks) but 64.1 -> 49.5 at K = 8960, M = 512, N = 1408 (16 of four or five). Up to
+//    16 k-blocks two groups do (K = 1024, M = 384, N = 4096: 16.5 -> 8.9 us, four groups 9.7).
 //  * more 64 x 128 tiles, up to two per CU: int4 takes 128 x 128 tiles of two groups while those
 //    fit one per CU (M = 256, N = 14336: 45.8 -> 35.1 us; bf16 M = 333, N = 7168 48.7 -> 38.7,
 //    64 x 128 tiles 45.0), otherwise, and for ternary, 64 x 128 tiles of two groups (M = 192, N =
@@ -1017,16 +1046,18 @@ bool choose_small_tiles(int fmt, const GemmDesc& d, int dtype, const PrefillLaun
   const bool int4 = fmt == HQ_FORMAT_INT4;
   const uint32_t t64 = make_launch(4, 1, d, 2).tiles, t128 = make_launch(8, 1, d, 2).tiles;
   if (t64 <= cus) {
-    // Tiles from which the whole tiles win, for 256 CUs.
+    // Tiles from which the whole tiles win, for 256 CUs, where their cost and the split's are too close to tell
+    // (1% of 18,500 shapes then take over 2% more than by the line alone, 27% less by as much), over a short K
+    // or where a workspace cap left the plan unsplit.
     uint32_t from = d.nkb <= 16u ? 32u : int4 && d.nkb > 32u ? 80u : 64u;
     if (d.nkb > 64u) from += int4 ? (d.nkb - 64u) / 2u : (d.nkb - 64u) * 7u / 5u;
-    if (int4 && dtype == HQ_DTYPE_BF16 && d.nkb > 24u)
-      from = d.nkb <= 40u ? 80u : std::min(240u, 88u + (std::max(d.nkb, 64u) - 64u) * 5u / 4u);
-    if (!int4 && d.nkb > 64u) from = std::max(from, dtype == HQ_DTYPE_BF16 ? 100u : std::min(136u, 3u * d.nkb - 136u));
-    if (!int4 && d.gen && d.nkb > 64u) from = std::max(136u, from * 9u / 8u);
-    if ((uint64_t)t64 * 256u < (uint64_t)from * cus) return false;
-    *out = make_whole(4, d.nkb <= 16u ? 2 : 4, 2, d);
-    return true;
+    bool whole = (uint64_t)t64 * 256u >= (uint64_t)from * cus;
+    if (d.nkb > 16u && cur.psk != 0u) {
+      const float r = whole_over_split(fmt, dtype, d, cur, t64, cus);
+      whole = r < 0.98f || (whole && r <= 1.04f);
+    }
+    if (whole) *out = make_whole(4, d.nkb <= 16u ? 2 : 4, 2, d);
+    return whole;
   }
   // A long K stays split over workgroups (K = 27648, M = 512, N = 5120: int4 170 us against 186-199), for
   // ternary, whose split is cheaper, already past 40 k-blocks (6144 x 5120, M = 400: 40.3 against 43.8

@@ -38,25 +38,11 @@ def test_row_tiles_by_type():
         assert f.split(" ws=")[1] == b.split(" ws=")[1]
 
 
-# Whole 64 x 128 prefill tiles against the K split over workgroups: from how many tiles, by K and type.
-@pytest.mark.parametrize("fmt,dt,M,kblocks,N,whole", [
-    (I4, BF16, 96, 28, 4608, False), (I4, F16, 96, 28, 4608, True), (I4, BF16, 128, 28, 5120, True),
-    (I4, BF16, 96, 64, 5120, False), (I4, F16, 96, 64, 5120, True), (I4, BF16, 96, 64, 6144, True),
-    (I4, BF16, 226, 98, 3456, False), (I4, BF16, 81, 112, 7168, False), (I4, F16, 81, 112, 7168, True),
-    (I4, BF16, 300, 216, 4096, False), (I4, BF16, 1024, 216, 1984, True),
-    (T2, F16, 226, 80, 3072, False), (T2, BF16, 192, 80, 4096, False), (T2, F16, 128, 80, 6656, True),
-    (T2, F16, 96, 88, 7936, False), (T2, F16, 333, 98, 2688, False), (T2, BF16, 333, 98, 2688, True), (T2, F16, 300, 64, 2048, True),
-])
-def test_small_prefill_tiles_by_type(fmt, dt, M, kblocks, N, whole):
-    assert ("64x128 tiles=" if whole else "whole=0 stream-K") in plan(fmt, dt, M, 128 * kblocks, N)
-
-
 # Ternary prefill in groups of 64 past one 64 x 128 tile per CU: the 64-row tiles stay where their rounds of
-# one tile per CU are cheaper, the K split over a long K.
+# one tile per CU are cheaper.
 @pytest.mark.parametrize("dt,group,M,kblocks,N,tile", [
     (BF16, 64, 643, 15, 23680, "64-row tiles=1023 whole"), (BF16, 64, 736, 17, 15360, "64-row tiles=720 whole"),
     (F16, 64, 736, 17, 15360, "128-row tiles=360"), (BF16, 64, 891, 46, 15360, "128-row tiles=420"),
-    (F16, 64, 144, 150, 7936, "whole=0 stream-K"), (BF16, 64, 300, 27, 7168, "64x128"),
 ])
 def test_ternary_tiles_past_one_per_cu(dt, group, M, kblocks, N, tile):
     d = plan(T2, dt, M, 128 * kblocks, N, group=group)

@@ -83,6 +83,26 @@ def test_default_plans(cuda, fmt, M, K, N, g, want):
         assert want in hq.describe(fmt, dt, M, K, N, group=g)
 
 
+# Whole 64 x 128 tiles against the K split over workgroups, by cost (the planner needs the device's occupancy for
+# the split): shapes measured 5% and more apart, where K divides well, badly, and with ragged rows.
+@pytest.mark.parametrize("fmt,dt,group,M,kblocks,N,whole", [
+    (O.INT4, O.BF16, 128, 81, 112, 7168, False), (O.INT4, O.BF16, 128, 300, 216, 4096, False), (O.INT4, O.BF16, 128, 512, 70, 1408, True),
+    (O.INT4, O.BF16, 128, 768, 160, 2176, True), (O.INT4, O.F16, 128, 81, 112, 7168, True), (O.INT4, O.F16, 128, 96, 64, 5120, True),
+    (O.TERNARY2, O.F16, 128, 226, 80, 3072, False), (O.TERNARY2, O.F16, 128, 226, 76, 2560, True),
+    (O.TERNARY2, O.BF16, 128, 81, 76, 5120, True), (O.TERNARY2, O.F16, 128, 300, 64, 2048, True),
+    (O.TERNARY2, O.BF16, 128, 747, 128, 461, True), (O.TERNARY2, O.BF16, 64, 300, 27, 2048, True),
+    (O.INT4, O.BF16, 32, 1024, 200, 1792, True),
+])
+def test_small_tiles_by_cost(cuda, fmt, dt, group, M, kblocks, N, whole):
+    import torch
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the boundaries are those of a 256-CU device")
+    d = hq.describe(fmt, dt, M, 128 * kblocks, N, group=group, with_bias=group == 32)
+    assert ("64x128 tiles=" if whole else "whole=0 stream-K") in d, d
+    assert d.split(" ws=")[1] == hq.describe(fmt, O.F16 + O.BF16 - dt, M, 128 * kblocks, N, group=group, with_bias=group == 32).split(" ws=")[1]
+
+
 # Three equal pieces along K (the planner needs the device's occupancy for them): ternary fp16, and both
 # types in groups of 64, stay split; pieces that do not come out equal take the whole tiles.
 @pytest.mark.parametrize("dt,group,M,kblocks,N,split", [
